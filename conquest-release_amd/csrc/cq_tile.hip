@@ -1,4 +1,4 @@
-// Output-tile schedule and FP64 tile kernel for uniform block sizes.
+// Output-tile schedules and their product kernels.
 //
 // The same block products as the triplet kernels (m_kern_max / m_kern_min,
 // src/multiply_kernel_default.f90:204-214 and :392-402), grouped so that
@@ -12,21 +12,22 @@
 //  * an entry of a tile is one contraction atom x with its (up to 8) left
 //    operand blocks P(row, x) and (up to 8) right operand blocks Q(column, x);
 //    entries of a tile are in ascending x (type 1: the reference's k order);
-//  * one workgroup (4 wavefronts, three workgroups per CU) runs one tile.
-//    Chunks of entries have their operand blocks copied HBM->LDS
-//    (global_load_lds, no registers) into one of two stages while the
+//  * uniform 9, 13, 16: each 4x4-block quadrant of a tile is the work of one
+//    wavefront of its own, driven by a list of records (k_wave_products);
+//  * the other kernels run a tile with one workgroup (4 wavefronts, three
+//    workgroups per CU). Chunks of entries have their operand blocks copied
+//    HBM->LDS (global_load_lds, no registers) into one of two stages while the
 //    previous chunk is computed from the other (one barrier per chunk); each
-//    wavefront accumulates 16 output blocks of the tile with
-//    v_mfma_f64_16x16x4 from LDS and finally writes each of them once (zeros
-//    where a block has no products), so the output is fully overwritten as
-//    mat_mult overwrites it (src/multiply_module.f90:204-208). Ownership is a
-//    Latin square (two blocks per tile row and column per wavefront), chosen
-//    when the plan is built to balance the wavefronts' product counts;
-//  * the plan holds each wavefront's products of each chunk as a list of
-//    packed LDS offsets (left | right << 16, in elements), sorted by the
-//    wavefront's output block and, within a block, by entry, with the count per
-//    block in one 64-bit word (16 x 4 bits). The kernel walks that list: no
-//    product discovery at run time.
+//    wavefront accumulates 16 output blocks of the tile with MFMA from LDS.
+//    Mixed sizes: ownership is a Latin square (two blocks per tile row and
+//    column per wavefront), chosen when the plan is built to balance the
+//    wavefronts' product counts, and the plan holds each wavefront's products
+//    of each chunk as a list of packed LDS offsets sorted by the wavefront's
+//    output block and, within a block, by entry, with the count per block in
+//    one 64-bit word (16 x 4 bits): no product discovery at run time;
+//  * every output block is written once (zeros where it has no products), so
+//    the output is fully overwritten as mat_mult overwrites it
+//    (src/multiply_module.f90:204-208).
 // Summation order per output block is fixed (ascending x), so results are
 // bitwise reproducible run to run.
 #include <hip/hip_runtime.h>
@@ -64,6 +65,35 @@ __device__ inline s16x4 pack_bf16_hi(const uint32_t w[4]) {
   return __builtin_bit_cast(s16x4, (uint64_t)x | ((uint64_t)y << 32));
 }
 
+// In place: split-BF16 words of contraction indices 4g..4g+3 (indices >= NSF
+// zeroed) -> the hi (registers 0, 1) and lo (2, 3) operands of
+// v_mfma_f32_16x16x16_bf16.
+template <int NSF>
+__device__ inline void split_words(float *k, int g) {
+  uint32_t x[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) x[i] = (NSF < 16 && 4 * g + i >= NSF) ? 0u : __float_as_uint(k[i]);
+  k[0] = __uint_as_float(__builtin_amdgcn_perm(x[1], x[0], 0x05040100u));
+  k[1] = __uint_as_float(__builtin_amdgcn_perm(x[3], x[2], 0x05040100u));
+  k[2] = __uint_as_float(__builtin_amdgcn_perm(x[1], x[0], 0x07060302u));
+  k[3] = __uint_as_float(__builtin_amdgcn_perm(x[3], x[2], 0x07060302u));
+}
+__device__ inline s16x4 half_of(const float *k, int i) {
+  return __builtin_bit_cast(s16x4, (uint64_t)__float_as_uint(k[i]) | ((uint64_t)__float_as_uint(k[i + 1]) << 32));
+}
+
+// Lane N of each row of 16 lanes, for all lanes of that row.
+template <int N>
+__device__ inline float row_bcast(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + N, 0xf, 0xf, true));
+}
+template <int N>
+__device__ inline double row_bcast(double x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x150 + N, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x150 + N, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
 constexpr int kWaves = 4;                    // wavefronts per workgroup (one tile)
 constexpr int kTileThreads = 64 * kWaves;
 constexpr int kSlots = 64 / kWaves;          // output blocks per wavefront
@@ -86,13 +116,6 @@ constexpr int kDenseEntries = 64;            // entries per chunk at most there 
 constexpr int stage_cap(int nsf) {
   return kStageBytes / (nsf * nsf * 8) > 16 ? kStageBytes / (nsf * nsf * 8) : 16;
 }
-
-template <int NSF>
-struct TileCfg {
-  static constexpr int NS2 = NSF * NSF;
-  static constexpr int CAP = stage_cap(NSF);
-  static constexpr int KS = (NSF + 3) / 4;              // MFMA k-steps per product
-};
 
 int tile_cap(int nsf) { return stage_cap(nsf); }
 
@@ -186,233 +209,313 @@ __device__ inline int64_t readlane64(int64_t v, int k) {
 // MODE 1: FP32 operands, v_mfma_f32_16x16x4, FP32 accumulation.
 // MODE 2: FP32 operands and MFMA, each product's result added into FP64
 //         registers (accumulator D[4(l/16)+e][l%16]).
-// MODE 3: FP32 operands and MFMA; the products of one output block within a
-//         chunk (consecutive in the wavefront's list, at most 15) chain in one
-//         FP32 accumulator, which is then added into the block's FP64 registers.
-// Pipeline per chunk c (one barrier): wait for chunk c's copies and the
-// prefetched registers, issue chunk c+1's copies into the other stage and the
-// register loads of chunk c+1's product list and chunk c+2's operand list,
-// then compute chunk c from LDS.
-template <int MODE, bool QT, int NSF, class ARG>
-__global__ void __launch_bounds__(kTileThreads) k_tile_products(
-    const ARG arg) {
+// MODE 4: split-BF16 words, three v_mfma_f32_16x16x16_bf16 per product, each
+//         product's FP32 sum added into FP64 registers.
+//
+// Operand registers of one NSF x NSF block, as the lane (r, g) = (l%16, l/16)
+// supplies them to the matrix instruction.
+template <int MODE, int NSF>
+struct Frag {
   using T = typename std::conditional<MODE == 0, double, float>::type;
-  using C = TileCfg<NSF>;
-  constexpr int STAGE = C::CAP * C::NS2 + kLdsPad * (int)(8 / sizeof(T));
-  __shared__ T stage0[STAGE];
-  __shared__ T stage1[STAGE];
+  static constexpr int KS = (NSF + 3) / 4;               // k-steps of 4 contraction indices
+  static constexpr bool R1 = MODE != 4 && NSF % 4 == 1;  // the last contraction index on the VALU
+  static constexpr int KM = MODE == 4 ? 4 : (R1 ? KS - 1 : KS);  // registers of the matrix steps
+  static_assert(NSF % 4 <= 1, "block sizes 4m and 4m + 1");
+  T k[KM];    // element of each matrix step (MODE 4: hi and lo operands, two registers each)
+  T last[4];  // R1: left, A[row][NSF-1] of the lane's 4 accumulator rows; right, B[NSF-1][r] in last[0]
+};
+
+// A block's bytes go to LDS 16 per lane; where they end inside the last lane's
+// 16, that lane takes the block's last 16 bytes instead, so the last element
+// lies wave_shift elements further than its index says (a copy instruction of
+// its own for the 4 or 8 bytes left would be the third of a 13x13 FP64 block).
+constexpr int wave_stride(int nsf, int size) { return (nsf * nsf * size + 15) / 16 * 16; }
+constexpr int wave_shift(int nsf, int size) { return (wave_stride(nsf, size) - nsf * nsf * size) / size; }
+
+// Element offsets in a block (as it lies in LDS) of a lane's operands: of its
+// first register (MODE 4: of each) and of the last contraction index. Lanes
+// beyond the block's rows, columns or indices read an element that feeds only
+// results that are not written.
+template <int MODE, bool RIGHT, bool QT, int NSF>
+struct FragOff {
+  using F = Frag<MODE, NSF>;
+  static constexpr bool KMAJ = RIGHT && !QT;   // contraction index fastest
+  static constexpr int N = MODE == 4 ? 4 : 1;
+  static constexpr int END = NSF * NSF - 1, SHIFT = wave_shift(NSF, MODE == 0 ? 8 : 4);
+  static_assert(SHIFT == 0 || (NSF % 4 == 1 && SHIFT == (MODE == 0 ? 1 : 3)), "only the last element is shifted");
+  int first[N], last;
+  __device__ inline FragOff(int r, int g) {
+    const int n = min(r, NSF - 1);
+    auto at = [](int i) { return i == END ? i + SHIFT : i; };
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int k = MODE == 4 ? min(4 * g + i, NSF - 1) : g;
+      first[i] = at(KMAJ ? k + NSF * n : n + NSF * k);
+    }
+    if (RIGHT) last = at(QT ? n + NSF * (NSF - 1) : NSF - 1 + NSF * n);
+    // Accumulator rows: FP64 g + 4e (load() shifts row NSF - 1), FP32 4g + e.
+    else last = MODE == 0 ? NSF * (NSF - 1) + g : at(NSF * (NSF - 1) + 4 * g);
+  }
+  template <class T>
+  __device__ inline void load(const T *blk, int g, F &f) const {
+    constexpr int STEP = KMAJ ? 4 : 4 * NSF;
+#pragma unroll
+    for (int i = 0; i < F::KM; ++i) f.k[i] = blk[first[N == 1 ? 0 : i] + (N == 1 ? STEP * i : 0)];
+    if constexpr (F::R1) {
+#pragma unroll
+      for (int e = 0; e < (RIGHT ? 1 : 4); ++e)
+        f.last[e] = blk[last + (MODE == 0 ? 4 * e + (!RIGHT && 4 * e == NSF - 1 ? SHIFT : 0) : e)];
+    }
+    if constexpr (MODE == 4) split_words<NSF>(f.k, g);
+  }
+};
+
+// Ring of operand blocks of a wavefront: what its share of the 160 KB LDS
+// holds beside the record words, with 2 wavefronts per SIMD (FP64) or 3.
+constexpr int kWaveWords = 256;  // record words in LDS
+constexpr int wave_per_simd(int mode) { return mode == 0 ? 2 : 3; }
+constexpr int wave_dmas(int nsf, int size) { return (nsf * nsf * size + 1023) / 1024; }  // copies per block
+constexpr int wave_ring(int mode, int nsf) {
+  const int size = mode == 0 ? 8 : 4;
+  const int r = ((mode == 0 ? 20480 : 12800) - 4 * kWaveWords) / wave_stride(nsf, size);
+  const int v = 63 / wave_dmas(nsf, size);  // the wait counts at most 63 copies
+  return (r < v ? r : v) < 28 ? (r < v ? r : v) : 28;
+}
+
+// One operand block from memory to LDS. `lane16`: 16 * lane, and `end16` that of
+// the last copy (its last lane takes the block's last 16 bytes); opaque, so that
+// they stay 32-bit offsets from the scalar block address.
+template <int BYTES>
+__device__ inline void dma_block(const char *src, char *dst, uint32_t &lane16, uint32_t &end16, int lane) {
+  constexpr int LANES = (BYTES + 15) / 16, N = (LANES + 63) / 64, REST = LANES - 64 * (N - 1);
+  auto d = (__attribute__((address_space(3))) void *)dst;
+  if constexpr (N > 1) {
+    asm volatile("" : "+v"(lane16));
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(src + lane16), d, 16, 0, 0);
+  }
+  static_assert(N <= 2, "blocks of at most 2 KB");
+  if (REST == 64 || lane < REST) {
+    asm volatile("" : "+v"(end16));
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(src + end16), d, 16,
+                                     1024 * (N - 1), 0);
+  }
+}
+
+// Waits until at most `after` blocks of PER copies each are in flight, `after`
+// rounded down to N, N/2, .., 4 or 0.
+template <int PER, int N>
+__device__ inline void wait_blocks(int32_t after) {
+  constexpr int v = N < 4 ? 0 : PER * N;
+  __builtin_amdgcn_s_waitcnt((v & 15) | (v >> 4 << 14) | 0xf70);  // vmcnt only
+  if constexpr (N >= 4) {
+    if (after < N) wait_blocks<PER, N / 2>(after);
+  }
+}
+
+// Uniform block sizes 9, 13, 16: one wavefront computes 4x4 output blocks (a
+// quadrant of a tile) in 16 accumulators, on its own: no barrier, no other
+// wavefront to wait for. Its records (contraction atoms, ascending) list the
+// present blocks of 4 rows and 4 columns. The blocks of the next records are
+// copied memory -> LDS into a ring while the oldest record's products run from
+// registers: every operand element is read from LDS once per record, and every
+// present pair with an output block is a bit test and the matrix steps.
+//
+// What bounds it (gfx950): a VALU instruction holds the SIMD as a matrix
+// instruction does (3 f64 MFMA take 217 cycles, with 16 VALU instructions of any
+// wavefront between them 292), so a product costs its matrix steps plus 4.6
+// cycles per VALU instruction, and the design keeps these few; what is left
+// is the scalar work and the branches of a record (about 1500 cycles of one
+// wavefront) and, at thousands of atoms, the copies beyond L2 (4096 atoms 13x13,
+// type 2: copies alone 34.5 ms, everything but the copies 37.5 ms).
+// Against one workgroup per 8x8 tile with its four wavefronts in step (a barrier
+// per chunk; the busiest wavefront has 1.25 to 1.56 times the mean products):
+// 13x13 FP64 4096 atoms type 2 50.2 -> 46.0 ms, 1024 atoms symmetric
+// 15.9 -> 15.3 ms, 9x9 FP32 with FP64 sums 1500 atoms 11.1 -> 8.9 ms, 13x13 split
+// BF16 1024 atoms 5.9 -> 5.0 ms, 9x9 FP64 60 atoms (one LNV solve) 12.5 -> 10.0 ms.
+// Tried and slower: operands straight to registers (4096 atoms 58 ms: 18 to 33
+// address cycles per load), two stages instead of the ring (split BF16 6.2 ms),
+// three wavefronts per SIMD with right operands read per product (9x9 11.1 ms).
+//
+// NSF = 4m + 1: the last contraction index is a rank-1 update on the VALU (four
+// fused multiply-adds after the matrix steps; a matrix step with three zeroed
+// indices takes 72 cycles in FP64).
+template <int MODE, bool QT, int NSF, class ARG>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(wave_per_simd(MODE))))
+k_wave_products(const ARG arg) {
+  using F = Frag<MODE, NSF>;
+  using T = typename F::T;
+  constexpr int NS2 = NSF * NSF;
+  constexpr int BYTES = NS2 * (int)sizeof(T);
+  constexpr int LB = wave_stride(NSF, (int)sizeof(T));
+  constexpr int RING = wave_ring(MODE, NSF), PER = wave_dmas(NSF, (int)sizeof(T));
+  static_assert(RING >= 8, "the ring holds every record");
+  __shared__ __attribute__((aligned(16))) char lds[RING * LB + 4 * kWaveWords];
   TileArgs a;
   const int32_t tile = tile_select(arg, a);
-  if (tile < 0) return;  // the whole workgroup leaves together
-  const int32_t *__restrict__ tile_chunk = a.tile_chunk;
-  const int64_t *__restrict__ chunk_lbeg = a.chunk_lbeg;
-  const int32_t *__restrict__ list = a.list;
-  const int64_t *__restrict__ pstart = a.pstart;
-  const uint64_t *__restrict__ pcnt = a.pcnt;
-  const uint32_t *__restrict__ prod = a.prod;
-  const int32_t *__restrict__ wave_out = a.wave_out;
-  const T *__restrict__ P = static_cast<const T *>(a.P);
-  const T *__restrict__ Q = static_cast<const T *>(a.Q);
+  if (tile < 0) return;
+  const int lane = threadIdx.x, r = lane & 15, g = lane >> 4;
+  const char *P = static_cast<const char *>(a.P), *Q = static_cast<const char *>(a.Q);
   T *__restrict__ O = static_cast<T *>(a.O);
-  const int tid = threadIdx.x;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63, r = lane & 15, g = lane >> 4;
-  constexpr int SA = 4 * NSF;             // A offset step per k-step
-  constexpr int SB = QT ? 4 * NSF : 4;    // B offset step per k-step
-  constexpr int REM = NSF - 4 * (C::KS - 1);  // valid g at the last k-step
-  const int oA = r + NSF * g;
-  const int oB = QT ? (r + NSF * g) : (g + NSF * r);
-  const bool last_ok = g < REM;
-  // The wavefront's output blocks (-1: none), set when the plan was built.
-  const int32_t *wo = wave_out + ((int64_t)tile * kWaves + w) * kSlots;
-  int32_t oblk[kSlots];
+  // The tile's output blocks (-1: none): bit 4*row + column of `valid`.
+  const int32_t *wo = a.wave_out + (int64_t)tile * 16;
+  const uint32_t valid = (uint32_t)__ballot(wo[r] >= 0) & 0xffffu;
+  dbl4 a64[16];
+  flt4 a32[16];
 #pragma unroll
-  for (int u = 0; u < kSlots; ++u) oblk[u] = wo[u];
-  dbl4 a64[kSlots];
-  flt4 a32[kSlots];
-#pragma unroll
-  for (int u = 0; u < kSlots; ++u) {
+  for (int u = 0; u < 16; ++u) {
     a64[u] = dbl4{0.0, 0.0, 0.0, 0.0};
     a32[u] = flt4{0.f, 0.f, 0.f, 0.f};
   }
-  const int32_t c0 = tile_chunk[tile], c1 = tile_chunk[tile + 1];
-  if (c0 < c1) {
-    // Per-chunk data of the tile held in registers, 64 chunks at a time: lane
-    // l has chunk_lbeg and this wavefront's product-list start and counts of
-    // chunk wb + l (index clamped to c1). Vector loads, refilled after the
-    // compute of a chunk, so the loop has no scalar loads (a scalar load
-    // outstanding during the compute would make every LDS wait also wait for
-    // it).
-    int32_t wb = c0;
-    int32_t cc = min(wb + lane, c1);
-    int64_t wcl = chunk_lbeg[cc];
-    int64_t wps = pstart[(int64_t)cc * kWaves + w];
-    int64_t wpc = (int64_t)pcnt[(int64_t)cc * kWaves + w];
-    auto cl_at = [&](int32_t x) { return readlane64(wcl, min(x, c1) - wb); };
-    auto ps_at = [&](int32_t x) { return readlane64(wps, min(x, c1) - wb); };
-    auto pc_at = [&](int32_t x) { return (uint64_t)readlane64(wpc, min(x, c1) - wb); };
-    uint32_t pl;
-    int32_t lvn = 0;
-    {
-      const int64_t cl0 = cl_at(c0), cl1 = cl_at(c0 + 1);
-      const int32_t lv0 = load_chunk_list(list, cl0, (int32_t)(cl1 - cl0), w, lane);
-      issue_stage<NSF, T>(lv0, (int32_t)(cl1 - cl0), P, Q, stage0, w, lane);
-      pl = prod[ps_at(c0) + lane];
-      if (c0 + 1 < c1) lvn = load_chunk_list(list, cl1, (int32_t)(cl_at(c0 + 2) - cl1), w, lane);
-    }
-    for (int32_t c = c0; c < c1; ++c) {
-      __builtin_amdgcn_s_waitcnt(0);
-      __syncthreads();
-      const bool odd = ((c - c0) & 1) != 0;
-      const T *cur = odd ? stage1 : stage0;
-      const uint32_t plc = pl;
-      const uint64_t cnt = pc_at(c);
-      if (c + 1 < c1) {
-        const int64_t cl1 = cl_at(c + 1), cl2 = cl_at(c + 2);
-        issue_stage<NSF, T>(lvn, (int32_t)(cl2 - cl1), P, Q, odd ? stage0 : stage1, w, lane);
-        pl = prod[ps_at(c + 1) + lane];
-        if (c + 2 < c1) lvn = load_chunk_list(list, cl2, (int32_t)(cl_at(c + 3) - cl2), w, lane);
+  const int64_t w0 = a.pstart[tile];
+  const int32_t nw = (int32_t)(a.pstart[tile + 1] - w0);
+  {
+    const FragOff<MODE, false, QT, NSF> oP(r, g);
+    const FragOff<MODE, true, QT, NSF> oQ(r, g);
+    constexpr int LANES = (BYTES + 15) / 16, LAST = (LANES - 1) % 64;
+    uint32_t l4 = 4u * (uint32_t)lane, lane16 = 16u * (uint32_t)lane;
+    uint32_t end16 = lane16 - (lane == LAST ? (uint32_t)(LB - BYTES) : 0u);
+    // Record words: a record is rows present | columns present << 4, then the
+    // present blocks (left by row, right by column). They come to LDS in pieces
+    // of 64 words, three pieces ahead, and from there to a register of the
+    // lanes, word `i` of the list in lane i - base. A piece is first read at
+    // least 43 block copies after it was issued (65 words, two of three of them
+    // blocks), more than the ring's, so the waits for blocks cover it.
+    const char *words = (const char *)(a.prod + w0);
+    char *wring = lds + RING * LB;
+    auto piece = [&](int32_t j) {
+      if (64 * j >= nw) return;
+      asm volatile("" : "+v"(l4));
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(words + 256 * (int64_t)j + l4),
+                                       (__attribute__((address_space(3))) void *)(wring + 256 * (j & 3)), 4, 0, 0);
+    };
+    int32_t at = 0, base = 0;
+    uint32_t win;
+    auto refill = [&]() {
+      base = at;
+      win = ((const uint32_t *)wring)[(at + lane) % kWaveWords];
+    };
+    auto word = [&](int32_t i) { return (uint32_t)__builtin_amdgcn_readlane((int)win, i - base); };
+    for (int32_t j = 0; j < 4; ++j) piece(j);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0);
+    asm volatile("" ::: "memory");
+    refill();
+    uint64_t queue = 0;             // masks of the records in the ring, oldest in the low byte
+    int32_t nq = 0, held = 0;       // records, blocks in the ring
+    int32_t head = 0, tail = 0;     // LDS offsets of the oldest block and of the next free slot
+    uint32_t coming = nw > 0 ? word(0) : 0u;  // masks of the record at `at`, 0 past the last
+    auto fits = [&]() {
+      return (nq < 8) & (coming != 0) & (held + __builtin_popcount(coming) <= RING);
+    };
+    auto issue = [&]() {
+      const uint32_t m = coming;
+      held += __builtin_popcount(m);
+      queue |= (uint64_t)m << (8 * nq++);
+      ++at;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        if (!(m >> k & 1u)) continue;
+        dma_block<BYTES>((k < 4 ? P : Q) + (int64_t)word(at++) * BYTES, lds + tail, lane16, end16, lane);
+        tail = tail == (RING - 1) * LB ? 0 : tail + LB;
       }
-      int p = 0;
+      if (at + 9 > base + 64) {
+        const int32_t j = at >> 6;
+        if (j != base >> 6) piece(j + 3);
+        refill();
+      }
+      coming = at < nw ? word(at) : 0u;
+    };
+    while (fits()) issue();
+    if (nq > 0) do {
+      const uint32_t m = (uint32_t)queue & 0xffu;
+      const int32_t n = __builtin_popcount(m);
+      queue >>= 8;
+      --nq;
+      asm volatile("" ::: "memory");
+      wait_blocks<PER, (RING >= 20 ? 16 : 8)>(held - n);
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // no LDS read is pending here; the compiler takes note
+      asm volatile("" ::: "memory");
+      const uint32_t cols = m >> 4;
+      auto step = [&](int32_t &o, int32_t by) {
+        o += by * LB;
+        o = o >= RING * LB ? o - RING * LB : o;
+        o = __builtin_amdgcn_readfirstlane(o);
+      };
+      int32_t pq = head;
+      step(pq, __builtin_popcount(m & 15u));
+      F right[4];
 #pragma unroll
-      for (int u = 0; u < kSlots; ++u) {
-        const int n = (int)((cnt >> (4 * u)) & 15u);
-        flt4 run = {0.f, 0.f, 0.f, 0.f};  // MODE 3: this block's products of the chunk
-        for (int i = 0; i < n; ++i, ++p) {
-          const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)plc, p);
-          if constexpr (MODE == 4) {
-            // Split-BF16 x3: the whole contraction (NSF <= 16) in one K = 16
-            // step; lane (r, g) holds contraction indices 4g..4g+3 as four
-            // LDS words (bits 0-15 hi, 16-31 lo; indices >= NSF zeroed),
-            // repacked into the hi and lo operands of v_mfma_f32_16x16x16_bf16.
-            // hi.hi + hi.lo + lo.hi chain in FP32; each product's sum is
-            // added into the FP64 accumulator (D[4g + e][r]).
-            const T *la = cur + (int)(v & 0xffffu) + r + NSF * 4 * g;
-            const T *lq = cur + (int)(v >> 16) + (QT ? r + NSF * 4 * g : 4 * g + NSF * r);
-            uint32_t wa[4], wb[4];
+      for (int k = 0; k < 4; ++k) {
+        if (!(cols >> k & 1u)) continue;
+        oQ.load((const T *)(lds + pq), g, right[k]);
+        step(pq, 1);
+      }
+      F left[MODE == 0 ? 4 : 1];
+      if constexpr (MODE == 0) {
 #pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4) {
-              wa[i4] = __float_as_uint(la[NSF * i4]);
-              wb[i4] = __float_as_uint(lq[QT ? NSF * i4 : i4]);
-              if (NSF < 16 && 4 * g + i4 >= NSF) {
-                wa[i4] = 0u;
-                wb[i4] = 0u;
+        for (int u = 0; u < 4; ++u) {
+          if (!(m >> u & 1u)) continue;
+          oP.load((const T *)(lds + head), g, left[u]);
+          step(head, 1);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (!(m >> u & 1u)) continue;
+        if constexpr (MODE != 0) {
+          oP.load((const T *)(lds + head), g, left[0]);
+          step(head, 1);
+        }
+        const F &x = left[MODE == 0 ? u : 0];
+        const uint32_t todo = (valid >> (4 * u)) & cols;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          if (!(todo >> k & 1u)) continue;
+          const F &y = right[k];
+          if constexpr (MODE == 0) {
+            dbl4 &d = a64[4 * u + k];
+#pragma unroll
+            for (int i = 0; i < F::KM; ++i) d = __builtin_amdgcn_mfma_f64_16x16x4f64(x.k[i], y.k[i], d, 0, 0, 0);
+            if constexpr (F::R1) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) d[i] = __builtin_fma(x.last[i], y.last[0], d[i]);
+            }
+          } else {
+            flt4 t = MODE == 1 ? a32[4 * u + k] : flt4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (MODE == 4) {
+              t = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(half_of(x.k, 0), half_of(y.k, 0), t, 0, 0, 0);
+              t = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(half_of(x.k, 0), half_of(y.k, 2), t, 0, 0, 0);
+              t = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(half_of(x.k, 2), half_of(y.k, 0), t, 0, 0, 0);
+            } else {
+#pragma unroll
+              for (int i = 0; i < F::KM; ++i) t = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[i], y.k[i], t, 0, 0, 0);
+              if constexpr (F::R1) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) t[i] = __builtin_fmaf(x.last[i], y.last[0], t[i]);
               }
             }
-            const s16x4 ahi = pack_bf16_lo(wa), alo = pack_bf16_hi(wa);
-            const s16x4 bhi = pack_bf16_lo(wb), blo = pack_bf16_hi(wb);
-            flt4 t = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ahi, bhi, flt4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-            t = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(ahi, blo, t, 0, 0, 0);
-            t = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(alo, bhi, t, 0, 0, 0);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) a64[u][e] += (double)t[e];
-            continue;
-          }
-          if constexpr (REM == 1) {
-            // NSF = 4m + 1: the last contraction index k = NSF - 1 is a
-            // rank-1 update on the VALU, D[row][r] += A[row][k] * B[k][r]
-            // (one fused multiply-add per accumulator element, FP64 or FP32),
-            // instead of an MFMA step with three zeroed k (a quarter fewer
-            // MFMAs; accumulators in VGPRs, built with the VGPR MFMA form).
-            // Rows g+4e >= NSF read past the block (inside the stage and its
-            // pad) and only feed accumulator rows that are never written.
-            const T *la = cur + (int)(v & 0xffffu) + oA;
-            const T *lq = cur + (int)(v >> 16) + oB;
-            T a[C::KS - 1], bb[C::KS - 1];
-#pragma unroll
-            for (int s4 = 0; s4 < C::KS - 1; ++s4) {
-              a[s4] = la[SA * s4];
-              bb[s4] = lq[SB * s4];
-            }
-            // Accumulator rows: FP64 g+4e, FP32 4g+e.
-            const T *ca = cur + (int)(v & 0xffffu) + NSF * (NSF - 1) + (MODE == 0 ? g : 4 * g);
-            const T bl = QT ? cur[(int)(v >> 16) + NSF * (NSF - 1) + r] : cur[(int)(v >> 16) + (NSF - 1) + NSF * r];
-            T ce[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) ce[e] = ca[MODE == 0 ? 4 * e : e];
-            if constexpr (MODE == 0) {
-#pragma unroll
-              for (int s4 = 0; s4 < C::KS - 1; ++s4)
-                a64[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s4], bb[s4], a64[u], 0, 0, 0);
-#pragma unroll
-              for (int e = 0; e < 4; ++e) a64[u][e] = __builtin_fma(ce[e], bl, a64[u][e]);
-            } else if constexpr (MODE == 1) {
-#pragma unroll
-              for (int s4 = 0; s4 < C::KS - 1; ++s4)
-                a32[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s4], bb[s4], a32[u], 0, 0, 0);
-#pragma unroll
-              for (int e = 0; e < 4; ++e) a32[u][e] = __builtin_fmaf(ce[e], bl, a32[u][e]);
-            } else if constexpr (MODE == 3) {
-#pragma unroll
-              for (int s4 = 0; s4 < C::KS - 1; ++s4) run = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s4], bb[s4], run, 0, 0, 0);
-#pragma unroll
-              for (int e = 0; e < 4; ++e) run[e] = __builtin_fmaf(ce[e], bl, run[e]);
+            if constexpr (MODE == 1) {
+              a32[4 * u + k] = t;
             } else {
-              flt4 t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-              for (int s4 = 0; s4 < C::KS - 1; ++s4) t = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s4], bb[s4], t, 0, 0, 0);
-#pragma unroll
-              for (int e = 0; e < 4; ++e) a64[u][e] += (double)__builtin_fmaf(ce[e], bl, t[e]);
+              for (int i = 0; i < 4; ++i) a64[4 * u + k][i] += (double)t[i];
             }
-            continue;
-          }
-          const T *la = cur + (int)(v & 0xffffu) + oA;
-          const T *lq = cur + (int)(v >> 16) + oB;
-          T a[C::KS], bb[C::KS];
-#pragma unroll
-          for (int s4 = 0; s4 < C::KS; ++s4) {
-            a[s4] = la[SA * s4];
-            bb[s4] = lq[SB * s4];
-          }
-          if (REM < 4 && !last_ok) {
-            a[C::KS - 1] = (T)0;
-            bb[C::KS - 1] = (T)0;
-          }
-          if constexpr (MODE == 0) {
-#pragma unroll
-            for (int s4 = 0; s4 < C::KS; ++s4)
-              a64[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s4], bb[s4], a64[u], 0, 0, 0);
-          } else if constexpr (MODE == 1) {
-#pragma unroll
-            for (int s4 = 0; s4 < C::KS; ++s4)
-              a32[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s4], bb[s4], a32[u], 0, 0, 0);
-          } else if constexpr (MODE == 3) {
-#pragma unroll
-            for (int s4 = 0; s4 < C::KS; ++s4) run = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s4], bb[s4], run, 0, 0, 0);
-          } else {
-            flt4 t = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int s4 = 0; s4 < C::KS; ++s4) t = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s4], bb[s4], t, 0, 0, 0);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) a64[u][e] += (double)t[e];
-          }
-        }
-        if constexpr (MODE == 3) {
-          if (n > 0) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) a64[u][e] += (double)run[e];
           }
         }
       }
-      if (c + 4 > wb + 63 && c + 1 < c1) {  // next iteration reads up to chunk c + 3
-        wb = c + 1;
-        cc = min(wb + lane, c1);
-        wcl = chunk_lbeg[cc];
-        wps = pstart[(int64_t)cc * kWaves + w];
-        wpc = (int64_t)pcnt[(int64_t)cc * kWaves + w];
-      }
-    }
+      head = pq;
+      held -= n;
+      while (fits()) issue();
+    } while (nq > 0);
   }
-  if (r < NSF) {
 #pragma unroll
-    for (int u = 0; u < kSlots; ++u) {
-      if (oblk[u] < 0) continue;
-      T *o = O + (int64_t)oblk[u] * C::NS2;
+  for (int u = 0; u < 16; ++u) {
+    if (!(valid >> u & 1u)) continue;
+    T *o = O + (int64_t)wo[u] * NS2 + NSF * r;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int row = MODE == 0 ? g + 4 * e : 4 * g + e;
-        if (row < NSF) o[row + NSF * r] = MODE == 0 ? (T)a64[u][e] : (MODE == 1 ? (T)a32[u][e] : (T)a64[u][e]);
-      }
+    for (int i = 0; i < 4; ++i) {
+      const int row = MODE == 0 ? g + 4 * i : 4 * g + i;
+      if (r < NSF && row < NSF) o[row] = MODE == 1 ? (T)a32[u][i] : (T)a64[u][i];
     }
   }
 }
@@ -425,8 +528,9 @@ __global__ void __launch_bounds__(kTileThreads) k_tile_products(
 // such block. A block pair whose output block does not exist only feeds
 // accumulator elements that are never written; every output block sums its
 // products in entry (x) order, one fused step per product, as the triplet
-// kernel does. Same chunks, stages and copies as k_tile_products; the chunk's
-// entries (at most 64, one per lane) replace the product lists.
+// kernel does. Chunk c's copies are waited for (one barrier), chunk c+1's issued
+// into the other stage, then chunk c computed; the chunk's entries are at most
+// 64, one per lane.
 template <int MODE, bool QT, class ARG>
 __global__ void __launch_bounds__(kTileThreads) k_tile_dense4(
     const ARG arg) {
@@ -654,37 +758,25 @@ __device__ inline void entry_wave_counts(uint32_t m, const uint8_t *__restrict__
 }
 
 // Chunks of a tile: at most max_entries consecutive entries whose operand
-// blocks fit `cap` and (with an owner table) that give no wavefront more than
-// kWaveProducts products. With FILL unset, counts them; with FILL set, writes each chunk's
-// first entry.
+// blocks fit `cap`. With FILL unset, counts them; with FILL set, writes each
+// chunk's first entry.
 template <bool FILL>
-__global__ void k_chunks(const int32_t *__restrict__ tebeg, const uint32_t *__restrict__ mask,
-                         const uint8_t *__restrict__ owner, int32_t n_tiles, int32_t cap, int32_t max_entries,
-                         const int32_t *__restrict__ tchunk, int32_t *__restrict__ out) {
+__global__ void k_chunks(const int32_t *__restrict__ tebeg, const uint32_t *__restrict__ mask, int32_t n_tiles,
+                         int32_t cap, int32_t max_entries, const int32_t *__restrict__ tchunk,
+                         int32_t *__restrict__ out) {
   const int32_t t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n_tiles) return;
   int32_t nch = 0, sum = 0, ne = 0;
-  int wc[kWaves] = {};
   for (int32_t e = tebeg[t]; e < tebeg[t + 1]; ++e) {
-    const uint32_t m = mask[e];
-    const int32_t c = __popc(m);
-    int pw[kWaves] = {};
-    if (owner) entry_wave_counts(m, owner + (int64_t)t * 64, pw);  // no owner: no per-wavefront limit
-    bool over = false;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) over |= wc[w] + pw[w] > kWaveProducts;
-    if (nch == 0 || sum + c > cap || ne == max_entries || over) {
+    const int32_t c = __popc(mask[e]);
+    if (nch == 0 || sum + c > cap || ne == max_entries) {
       if (FILL) out[tchunk[t] + nch] = e;
       ++nch;
       sum = 0;
       ne = 0;
-#pragma unroll
-      for (int w = 0; w < kWaves; ++w) wc[w] = 0;
     }
     sum += c;
     ++ne;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) wc[w] += pw[w];
   }
   if (!FILL) out[t] = nch;
 }
@@ -696,66 +788,90 @@ __global__ void k_chunk_tile(const int32_t *__restrict__ tchunk, int32_t n_tiles
   for (int32_t c = tchunk[t]; c < tchunk[t + 1]; ++c) ctile[c] = t;
 }
 
-// Product lists of each chunk, sorted by (wavefront, slot, entry). Count pass
-// (FILL unset): products per chunk into np. Fill pass: with pbase = the
-// chunk's first product, writes pstart/pcnt of its wavefronts and the packed
-// LDS offsets (left | right << 16, elements) of every product.
+// Records of k_wave_products, one wavefront per quadrant q (src[q] = tile * 4 +
+// quadrant): of the tile's entries (ascending contraction atom) those with a
+// product in the quadrant; the rows and columns that have one, then their
+// block indices. A record holds at most `cap` blocks: an entry with more
+// becomes several records over the same columns, each with some of its rows
+// (cap >= 5). Count pass (FILL unset): words, products and blocks of each quadrant.
 template <bool FILL>
-__global__ void k_chunk_prods(int32_t nch, const int32_t *__restrict__ chunk_entry, const int32_t *__restrict__ ctile,
-                              const uint32_t *__restrict__ mask, const int32_t *__restrict__ coff,
-                              const uint8_t *__restrict__ owner, int32_t ns2, int64_t *__restrict__ np,
-                              const int64_t *__restrict__ pbase, int64_t *__restrict__ pstart,
-                              uint64_t *__restrict__ pcnt, uint32_t *__restrict__ prod) {
-  const int32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= nch) return;
-  const uint8_t *own = owner + (int64_t)ctile[c] * 64;
-  const int32_t e0 = chunk_entry[c], e1 = chunk_entry[c + 1];
-  uint8_t cnt[64];
-  for (int i = 0; i < 64; ++i) cnt[i] = 0;
-  int32_t tot = 0;
-  for (int32_t e = e0; e < e1; ++e) {
-    const uint32_t m = mask[e];
-    for (uint32_t ym = m & 0xffu; ym; ym &= ym - 1u) {
-      const int u = __builtin_ctz(ym);
-      for (uint32_t bm = (m >> 8) & 0xffu; bm; bm &= bm - 1u) {
-        const uint8_t o = own[u * 8 + __builtin_ctz(bm)];
-        if (o != 0xff) {
-          ++cnt[o];
-          ++tot;
-        }
+__global__ void __launch_bounds__(256) k_wave_records(
+    const int32_t *__restrict__ src, int32_t n_wave, int32_t cap, const int32_t *__restrict__ wave_out,
+    const int32_t *__restrict__ tebeg, const int32_t *__restrict__ ep, const int32_t *__restrict__ eq,
+    int64_t *__restrict__ nword, int64_t *__restrict__ nprod, int64_t *__restrict__ nload,
+    const int64_t *__restrict__ beg, uint32_t *__restrict__ out) {
+  const int lane = threadIdx.x & 63;
+  const int32_t q = (int32_t)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+  if (q >= n_wave) return;
+  const int32_t t = src[q] >> 2, w = src[q] & 3;
+  const int qr = 4 * (w >> 1), qc = 4 * (w & 1);
+  const uint32_t valid = (uint32_t)__ballot(wave_out[(int64_t)q * 16 + (lane & 15)] >= 0) & 0xffffu;
+  int64_t at = FILL ? beg[q] : 0;
+  int64_t prods = 0, loads = 0;
+  for (int32_t e0 = tebeg[t]; e0 < tebeg[t + 1]; e0 += 64) {
+    const int32_t e = e0 + lane;
+    int32_t b[8];
+    uint32_t rows = 0, cols = 0;
+    int np = 0;
+    if (e < tebeg[t + 1]) {
+      uint32_t pm = 0, qm = 0;
+      for (int k = 0; k < 4; ++k) {
+        b[k] = ep[(int64_t)e * 8 + qr + k];
+        b[4 + k] = eq[(int64_t)e * 8 + qc + k];
+        pm |= (uint32_t)(b[k] >= 0) << k;
+        qm |= (uint32_t)(b[4 + k] >= 0) << k;
+      }
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t c = (pm >> k & 1u) ? (valid >> (4 * k)) & qm : 0u;
+        np += __popc(c);
+        cols |= c;
+        rows |= (uint32_t)(c != 0) << k;
       }
     }
+    // The entry's rows in `parts` records of nearly equal size.
+    const int nr = __popc(rows), nc = __popc(cols);
+    const int per = cap - nc, parts = nr == 0 ? 0 : (nr + per - 1) / per;
+    const int len = parts * (1 + nc) + nr;
+    int before = len;  // inclusive prefix sum of the records' words over the lanes
+    for (int off = 1; off < 64; off <<= 1) {
+      const int v = __shfl_up(before, off, 64);
+      if (lane >= off) before += v;
+    }
+    if (FILL && parts > 0) {
+      int64_t o = at + before - len;
+      int done = 0;
+      for (int part = 0; part < parts; ++part) {
+        const int take = (nr - done + parts - part - 1) / (parts - part);
+        const int64_t head = o++;
+        uint32_t rm = 0;
+        int seen = 0;
+        for (int k = 0; k < 4; ++k)
+          if (rows >> k & 1u) {
+            if (seen >= done && seen < done + take) {
+              rm |= 1u << k;
+              out[o++] = (uint32_t)b[k];
+            }
+            ++seen;
+          }
+        for (int k = 0; k < 4; ++k)
+          if (cols >> k & 1u) out[o++] = (uint32_t)b[4 + k];
+        out[head] = rm | cols << 4;
+        done += take;
+      }
+    }
+    at += __shfl(before, 63, 64);
+    prods += np;
+    loads += nr + parts * nc;
   }
   if (!FILL) {
-    np[c] = tot;
-    return;
-  }
-  uint16_t off[64];
-  int32_t run = 0;
-  for (int w = 0; w < kWaves; ++w) {
-    pstart[(int64_t)c * kWaves + w] = pbase[c] + run;
-    uint64_t word = 0;
-    for (int l = 0; l < kSlots; ++l) {
-      off[w * kSlots + l] = (uint16_t)run;
-      run += cnt[w * kSlots + l];
-      word |= (uint64_t)cnt[w * kSlots + l] << (4 * l);
+    for (int off = 32; off > 0; off >>= 1) {
+      prods += __shfl_down(prods, off, 64);
+      loads += __shfl_down(loads, off, 64);
     }
-    pcnt[(int64_t)c * kWaves + w] = word;
-  }
-  for (int32_t e = e0; e < e1; ++e) {
-    const uint32_t m = mask[e];
-    const uint32_t ym = m & 0xffu, bmask = (m >> 8) & 0xffu;
-    const int32_t base = coff[e];
-    for (uint32_t yb = ym; yb; yb &= yb - 1u) {
-      const int u = __builtin_ctz(yb);
-      const uint32_t aoff = (uint32_t)((base + __popc(ym & ((1u << u) - 1u))) * ns2);
-      for (uint32_t bm = bmask; bm; bm &= bm - 1u) {
-        const int col = __builtin_ctz(bm);
-        const uint8_t o = own[u * 8 + col];
-        if (o == 0xff) continue;
-        const uint32_t boff = (uint32_t)((base + __popc(ym) + __popc(bmask & ((1u << col) - 1u))) * ns2);
-        prod[pbase[c] + off[o]++] = aoff | (boff << 16);
-      }
+    if (lane == 0) {
+      nword[q] = at;
+      nprod[q] = prods;
+      nload[q] = loads;
     }
   }
 }
@@ -1032,8 +1148,11 @@ __device__ inline void issue_stage_mx(uint64_t lv, uint32_t lls, int32_t nb, con
   }
 }
 
-// Mixed-size tile kernel: as k_tile_products with per-slot output dimensions
-// (wave_dim) and per-product contraction dimension (product word bits 24-27).
+// Mixed-size tile kernel: per-slot output dimensions (wave_dim) and per-product
+// contraction dimension (product word bits 24-27). Pipeline per chunk c (one
+// barrier): wait for chunk c's copies and the prefetched registers, issue chunk
+// c+1's copies into the other stage and the register loads of chunk c+1's
+// product list and chunk c+2's operand list, then compute chunk c from LDS.
 template <int MODE, bool QT, int STG, class ARG>
 __global__ void __launch_bounds__(kTileThreads) k_tile_mixed(
     const ARG arg) {
@@ -1635,10 +1754,9 @@ int launch_kind(int kind, const ARG &arg, int32_t n, int32_t wgs, hipStream_t s)
     case kKindMixedLarge: hipLaunchKernelGGL((k_tile_mixed<MODE, QT, kStgLarge, ARG>), dim3(gridx), blk, 0, s, arg); break;
     case kKindQuadSmall: hipLaunchKernelGGL((k_tile_quad<MODE, QT, kStgSmall, ARG>), dim3(gridx), blk, 0, s, arg); break;
     case kKindQuadLarge: hipLaunchKernelGGL((k_tile_quad<MODE, QT, kStgLarge, ARG>), dim3(gridx), blk, 0, s, arg); break;
-    case kKindUniform + 4: hipLaunchKernelGGL((k_tile_products<MODE, QT, 4, ARG>), dim3(gridx), blk, 0, s, arg); break;
-    case kKindUniform + 9: hipLaunchKernelGGL((k_tile_products<MODE, QT, 9, ARG>), dim3(gridx), blk, 0, s, arg); break;
-    case kKindUniform + 13: hipLaunchKernelGGL((k_tile_products<MODE, QT, 13, ARG>), dim3(gridx), blk, 0, s, arg); break;
-    case kKindUniform + 16: hipLaunchKernelGGL((k_tile_products<MODE, QT, 16, ARG>), dim3(gridx), blk, 0, s, arg); break;
+    case kKindUniform + 9: hipLaunchKernelGGL((k_wave_products<MODE, QT, 9, ARG>), dim3(gridx), dim3(64), 0, s, arg); break;
+    case kKindUniform + 13: hipLaunchKernelGGL((k_wave_products<MODE, QT, 13, ARG>), dim3(gridx), dim3(64), 0, s, arg); break;
+    case kKindUniform + 16: hipLaunchKernelGGL((k_wave_products<MODE, QT, 16, ARG>), dim3(gridx), dim3(64), 0, s, arg); break;
     default: return cq::set_errorf(CQMM_ERR_ARG, "tile products: kernel kind %d has no instance", kind);
   }
   return cq::hip_check(hipGetLastError(), "tile-product kernel launch");
@@ -1647,11 +1765,10 @@ int launch_kind(int kind, const ARG &arg, int32_t n, int32_t wgs, hipStream_t s)
 template <int MODE, bool QT, class ARG>
 int launch_uniform(int kind, const ARG &arg, int32_t n, hipStream_t s) {
   const unsigned gridx = 8u * (unsigned)((n + 7) / 8);
-  const dim3 blk(kTileThreads);
   switch (kind) {
-    case kKindUniform + 9: hipLaunchKernelGGL((k_tile_products<MODE, QT, 9, ARG>), dim3(gridx), blk, 0, s, arg); break;
-    case kKindUniform + 13: hipLaunchKernelGGL((k_tile_products<MODE, QT, 13, ARG>), dim3(gridx), blk, 0, s, arg); break;
-    case kKindUniform + 16: hipLaunchKernelGGL((k_tile_products<MODE, QT, 16, ARG>), dim3(gridx), blk, 0, s, arg); break;
+    case kKindUniform + 9: hipLaunchKernelGGL((k_wave_products<MODE, QT, 9, ARG>), dim3(gridx), dim3(64), 0, s, arg); break;
+    case kKindUniform + 13: hipLaunchKernelGGL((k_wave_products<MODE, QT, 13, ARG>), dim3(gridx), dim3(64), 0, s, arg); break;
+    case kKindUniform + 16: hipLaunchKernelGGL((k_wave_products<MODE, QT, 16, ARG>), dim3(gridx), dim3(64), 0, s, arg); break;
     default: return cq::set_errorf(CQMM_ERR_ARG, "tile products: kernel kind %d has no instance", kind);
   }
   return cq::hip_check(hipGetLastError(), "tile-product kernel launch");
@@ -1675,9 +1792,10 @@ int launch_any(int mode, bool qt, int kind, const ARG &arg, int32_t n, int32_t w
     case 3: return launch_kind<1, true, ARG>(kind, arg, n, wgs, s);
     case 4: return launch_kind<2, false, ARG>(kind, arg, n, wgs, s);
     case 5: return launch_kind<2, true, ARG>(kind, arg, n, wgs, s);
-    // Mode 3 has its own instance in the uniform-size kernel only.
-    case 6: return kind >= kKindUniform ? launch_kind<3, false, ARG>(kind, arg, n, wgs, s) : launch_kind<2, false, ARG>(kind, arg, n, wgs, s);
-    case 7: return kind >= kKindUniform ? launch_kind<3, true, ARG>(kind, arg, n, wgs, s) : launch_kind<2, true, ARG>(kind, arg, n, wgs, s);
+    // Mode 3 (a block's products of one chunk may be summed in FP32) runs as
+    // mode 2, which adds every product in FP64.
+    case 6: return launch_kind<2, false, ARG>(kind, arg, n, wgs, s);
+    case 7: return launch_kind<2, true, ARG>(kind, arg, n, wgs, s);
     // Split-BF16 x3 (mode 4) runs in the class-tile kernel and the fixed-size
     // kernels of 9x9, 13x13 and 16x16 blocks.
     case 8:
@@ -1708,7 +1826,7 @@ namespace cq {
 int launch_tile_products_f32(const TilePlan &tp, bool q_trans, const float *P, const float *Q, float *O, int mode,
                              hipStream_t s) {
   if (tp.n_tiles == 0) return CQMM_OK;
-  return launch_any(mode, q_trans, tile_kind(tp), tile_launch_args(tp, P, Q, O), tp.n_tiles, tp.wgs, s);
+  return launch_tile_args(tp, q_trans, mode, tile_launch_args(tp, P, Q, O), s);
 }
 
 TileArgs tile_launch_args(const TilePlan &tp, const void *P, const void *Q, void *O) {
@@ -1733,7 +1851,7 @@ TileArgs tile_launch_args(const TilePlan &tp, const void *P, const void *Q, void
   a.P = P;
   a.Q = Q;
   a.O = O;
-  a.n_tiles = tp.n_tiles;
+  a.n_tiles = tp.n_wave ? tp.n_wave : tp.n_tiles;
   a.tile_base = 0;
   return a;
 }
@@ -1950,27 +2068,36 @@ int build_tiles(const TileBuildInput &in, TilePlan &tp, hipStream_t s) {
                       "H2D tile_out")) ||
       (st = hip_check(hipStreamSynchronize(s), "tile_out")))
     return st;
-  DevBuf d_owner;
   tp.dense = in.nsf == kDenseNsf;
-  if (tp.dense) {
-    // Wavefront w computes quadrant (w / 2, w % 2) of the tile: rows
-    // 4*(w/2)..+3, columns 4*(w%2)..+3.
-    std::vector<int32_t> wave_out((size_t)in.n_tiles * 64, -1);
-    for (int64_t t = 0; t < in.n_tiles; ++t)
+  // Output blocks of the tiles' quadrants: quadrant (w / 2, w % 2) has rows
+  // 4*(w/2)..+3, columns 4*(w%2)..+3.
+  std::vector<int32_t> wave_out((size_t)in.n_tiles * 64, -1), src;
+  parallel_for(in.n_tiles, [&](int64_t b, int64_t e) {
+    for (int64_t t = b; t < e; ++t)
       for (int u = 0; u < 8; ++u)
         for (int c = 0; c < 8; ++c)
           wave_out[(t * kWaves + (u >> 2) * 2 + (c >> 2)) * 16 + (u & 3) * 4 + (c & 3)] = tout32[t * 64 + u * 8 + c];
-    if ((st = tp.wave_out.alloc(wave_out.size() * 4))) return st;
-    if ((st = hip_check(hipMemcpyAsync(tp.wave_out.p, wave_out.data(), wave_out.size() * 4, hipMemcpyHostToDevice, s),
-                        "H2D wave_out")) ||
-        (st = hip_check(hipStreamSynchronize(s), "wave_out")))
-      return st;
-  } else {
-    pt.mark("  tiles: tile_out");
-    if ((st = assign_slots(in, tp.tile_out.as<int32_t>(), d_owner, tp.wave_out, s))) return st;
+  });
+  if (!tp.dense) {
+    // Only the quadrants with output blocks are work.
+    src.reserve((size_t)in.n_tiles * kWaves);
+    for (int64_t q = 0; q < (int64_t)in.n_tiles * kWaves; ++q) {
+      bool any = false;
+      for (int k = 0; k < 16; ++k) any |= wave_out[q * 16 + k] >= 0;
+      if (!any) continue;
+      if ((int64_t)src.size() != q)
+        for (int k = 0; k < 16; ++k) wave_out[src.size() * 16 + k] = wave_out[q * 16 + k];
+      src.push_back((int32_t)q);
+    }
+    wave_out.resize(src.size() * 16);
+    tp.n_wave = (int32_t)src.size();
   }
-  const int32_t max_entries = (tp.dense || tp.quad) ? kDenseEntries : kChunkEntries;
-  pt.mark("  tiles: owners");
+  if ((st = tp.wave_out.alloc(wave_out.size() * 4))) return st;
+  if ((st = hip_check(hipMemcpyAsync(tp.wave_out.p, wave_out.data(), wave_out.size() * 4, hipMemcpyHostToDevice, s),
+                      "H2D wave_out")) ||
+      (st = hip_check(hipStreamSynchronize(s), "wave_out")))
+    return st;
+  pt.mark("  tiles: quadrants");
   // Sort the products by (tile, contraction atom).
   unsigned end_bit = 1;
   const uint64_t kmax = (uint64_t)in.n_tiles * (uint64_t)in.nx;
@@ -2024,17 +2151,54 @@ int build_tiles(const TileBuildInput &in, TilePlan &tp, hipStream_t s) {
       (st = hip_check(hipStreamSynchronize(s), "load count")))
     return st;
   tp.n_loads = nl;
-  if ((st = tp.list.alloc(nl * 4))) return st;
-  hipLaunchKernelGGL(k_list_fill, dim3(grid1(ne, 256)), dim3(256), 0, s, d_ep.as<int32_t>(), d_eq.as<int32_t>(),
-                     d_elbeg.as<int64_t>(), ne, tp.list.as<int32_t>());
-  // Chunks.
   DevBuf d_tebeg, d_nch;
   if ((st = d_tebeg.alloc(((size_t)in.n_tiles + 1) * 4)) || (st = d_nch.alloc((size_t)in.n_tiles * 4))) return st;
   hipLaunchKernelGGL(k_tile_ebeg, dim3(grid1((int64_t)in.n_tiles + 1, 256)), dim3(256), 0, s, d_etile.as<int32_t>(), ne,
                      in.n_tiles, d_tebeg.as<int32_t>());
+  if (!tp.dense) {
+    // Entry records of the quadrants: count, first record of each, fill.
+    const size_t nq = src.size();
+    DevBuf d_src, d_nrec, d_nprod, d_nload;
+    if ((st = d_src.alloc(nq * 4)) || (st = d_nrec.alloc(nq * 8)) || (st = d_nprod.alloc(nq * 8)) ||
+        (st = d_nload.alloc(nq * 8)) || (st = tp.pstart.alloc((nq + 1) * 8)))
+      return st;
+    if ((st = hip_check(hipMemcpyAsync(d_src.p, src.data(), nq * 4, hipMemcpyHostToDevice, s), "H2D quadrants"))) return st;
+    const dim3 grid(grid1((int64_t)nq, 4));
+    hipLaunchKernelGGL((k_wave_records<false>), grid, dim3(256), 0, s, d_src.as<int32_t>(), tp.n_wave,
+                       8, tp.wave_out.as<int32_t>(), d_tebeg.as<int32_t>(), d_ep.as<int32_t>(), d_eq.as<int32_t>(),
+                       d_nrec.as<int64_t>(), d_nprod.as<int64_t>(), d_nload.as<int64_t>(), nullptr, nullptr);
+    int64_t nrec = 0, nprod = 0, nload = 0;
+    if ((st = hip_check(hipMemsetAsync(tp.pstart.p, 0, 8, s), "memset pstart")) ||
+        (st = inclusive_scan(d_nrec.as<int64_t>(), tp.pstart.as<int64_t>() + 1, nq, s)) ||
+        (st = inclusive_scan(d_nprod.as<int64_t>(), d_nprod.as<int64_t>(), nq, s)) ||
+        (st = inclusive_scan(d_nload.as<int64_t>(), d_nload.as<int64_t>(), nq, s)) ||
+        (st = hip_check(hipMemcpyAsync(&nrec, tp.pstart.as<int64_t>() + nq, 8, hipMemcpyDeviceToHost, s), "D2H records")) ||
+        (st = hip_check(hipMemcpyAsync(&nprod, d_nprod.as<int64_t>() + nq - 1, 8, hipMemcpyDeviceToHost, s), "D2H products")) ||
+        (st = hip_check(hipMemcpyAsync(&nload, d_nload.as<int64_t>() + nq - 1, 8, hipMemcpyDeviceToHost, s), "D2H loads")) ||
+        (st = hip_check(hipStreamSynchronize(s), "entry records")))
+      return st;
+    tp.n_prod = nprod;
+    tp.n_loads = nload;
+    if (nprod != n)
+      return set_errorf(CQMM_ERR_STATE, "tile plan: %lld listed products for %lld triplets", (long long)nprod,
+                        (long long)n);
+    // The kernel reads 64 words at a time.
+    if ((st = tp.prod.alloc(((size_t)nrec + 64) * 4))) return st;
+    if ((st = hip_check(hipMemsetAsync(tp.prod.as<uint32_t>() + nrec, 0, 64 * 4, s), "memset records tail"))) return st;
+    hipLaunchKernelGGL((k_wave_records<true>), grid, dim3(256), 0, s, d_src.as<int32_t>(), tp.n_wave,
+                       8, tp.wave_out.as<int32_t>(), d_tebeg.as<int32_t>(), d_ep.as<int32_t>(), d_eq.as<int32_t>(),
+                       nullptr, nullptr, nullptr, tp.pstart.as<int64_t>(), tp.prod.as<uint32_t>());
+    if ((st = hip_check(hipGetLastError(), "tile builder launch"))) return st;
+    st = hip_check(hipStreamSynchronize(s), "tile build");
+    pt.mark("  tiles: entry records");
+    return st;
+  }
+  if ((st = tp.list.alloc(nl * 4))) return st;
+  hipLaunchKernelGGL(k_list_fill, dim3(grid1(ne, 256)), dim3(256), 0, s, d_ep.as<int32_t>(), d_eq.as<int32_t>(),
+                     d_elbeg.as<int64_t>(), ne, tp.list.as<int32_t>());
+  // Chunks.
   hipLaunchKernelGGL((k_chunks<false>), dim3(grid1(in.n_tiles, 256)), dim3(256), 0, s, d_tebeg.as<int32_t>(),
-                     d_emask.as<uint32_t>(), d_owner.as<uint8_t>(), in.n_tiles, cap, max_entries, nullptr,
-                     d_nch.as<int32_t>());
+                     d_emask.as<uint32_t>(), in.n_tiles, cap, kDenseEntries, nullptr, d_nch.as<int32_t>());
   if ((st = tp.tile_chunk.alloc(((size_t)in.n_tiles + 1) * 4))) return st;
   if ((st = hip_check(hipMemsetAsync(tp.tile_chunk.p, 0, 4, s), "memset tile_chunk"))) return st;
   if ((st = inclusive_scan(d_nch.as<int32_t>(), tp.tile_chunk.as<int32_t>() + 1, (size_t)in.n_tiles, s))) return st;
@@ -2047,8 +2211,8 @@ int build_tiles(const TileBuildInput &in, TilePlan &tp, hipStream_t s) {
   DevBuf d_centry;
   if ((st = d_centry.alloc(((size_t)nch + 1) * 4))) return st;
   hipLaunchKernelGGL((k_chunks<true>), dim3(grid1(in.n_tiles, 256)), dim3(256), 0, s, d_tebeg.as<int32_t>(),
-                     d_emask.as<uint32_t>(), d_owner.as<uint8_t>(), in.n_tiles, cap, max_entries,
-                     tp.tile_chunk.as<int32_t>(), d_centry.as<int32_t>());
+                     d_emask.as<uint32_t>(), in.n_tiles, cap, kDenseEntries, tp.tile_chunk.as<int32_t>(),
+                     d_centry.as<int32_t>());
   if ((st = hip_check(hipMemcpyAsync(d_centry.as<int32_t>() + nch, &ne32, 4, hipMemcpyHostToDevice, s),
                       "H2D chunk end")))
     return st;
@@ -2059,61 +2223,19 @@ int build_tiles(const TileBuildInput &in, TilePlan &tp, hipStream_t s) {
   hipLaunchKernelGGL(k_entry_coff, dim3(grid1((int64_t)nch, 256)), dim3(256), 0, s, d_centry.as<int32_t>(),
                      d_elbeg.as<int64_t>(), (int64_t)nch, d_ecoff.as<int32_t>());
   pt.mark("  tiles: entries + chunks");
-  if (tp.dense) {
-    // The dense kernel reads the entries themselves; no product lists.
-    tp.chunk_entry = std::move(d_centry);
-    tp.entry_mask = std::move(d_emask);
-    tp.entry_coff = std::move(d_ecoff);
-    tp.n_prod = n;
-    if ((st = hip_check(hipGetLastError(), "tile builder launch"))) return st;
-    return hip_check(hipStreamSynchronize(s), "tile build");
-  }
-  // Product lists: count per chunk, first product of each chunk, fill.
-  DevBuf d_ctile, d_np, d_pbase;
-  if ((st = d_ctile.alloc((size_t)std::max(nch, 1) * 4)) || (st = d_np.alloc((size_t)std::max(nch, 1) * 8)) ||
-      (st = d_pbase.alloc(((size_t)nch + 1) * 8)))
-    return st;
-  hipLaunchKernelGGL(k_chunk_tile, dim3(grid1(in.n_tiles, 256)), dim3(256), 0, s, tp.tile_chunk.as<int32_t>(),
-                     in.n_tiles, d_ctile.as<int32_t>());
-  hipLaunchKernelGGL((k_chunk_prods<false>), dim3(grid1(std::max(nch, 1), 256)), dim3(256), 0, s, nch,
-                     d_centry.as<int32_t>(), d_ctile.as<int32_t>(), d_emask.as<uint32_t>(), d_ecoff.as<int32_t>(),
-                     d_owner.as<uint8_t>(), (int32_t)ns2, d_np.as<int64_t>(), nullptr, nullptr, nullptr, nullptr);
-  if ((st = hip_check(hipMemsetAsync(d_pbase.p, 0, 8, s), "memset pbase"))) return st;
-  if ((st = inclusive_scan(d_np.as<int64_t>(), d_pbase.as<int64_t>() + 1, (size_t)nch, s))) return st;
-  int64_t nprod = 0;
-  if ((st = hip_check(hipMemcpyAsync(&nprod, d_pbase.as<int64_t>() + nch, 8, hipMemcpyDeviceToHost, s), "D2H products")) ||
-      (st = hip_check(hipStreamSynchronize(s), "product count")))
-    return st;
-  tp.n_prod = nprod;
-  if (nprod != n)
-    return set_errorf(CQMM_ERR_STATE, "tile plan: %lld listed products for %lld triplets", (long long)nprod,
-                      (long long)n);
-  // pstart/pcnt carry one extra chunk (the clamp target of the kernel's
-  // per-chunk registers) and prod kWaveProducts extra entries (each
-  // wavefront loads a full row of 64 list words per chunk).
-  if ((st = tp.pstart.alloc(((size_t)nch + 1) * kWaves * 8)) || (st = tp.pcnt.alloc(((size_t)nch + 1) * kWaves * 8)) ||
-      (st = tp.prod.alloc(((size_t)nprod + kWaveProducts) * 4)))
-    return st;
-  std::vector<int64_t> tail_start(kWaves, nprod);
-  if ((st = hip_check(hipMemsetAsync(tp.pcnt.as<uint64_t>() + (size_t)nch * kWaves, 0, kWaves * 8, s), "memset pcnt")) ||
-      (st = hip_check(hipMemcpyAsync(tp.pstart.as<int64_t>() + (size_t)nch * kWaves, tail_start.data(), kWaves * 8,
-                                     hipMemcpyHostToDevice, s), "H2D pstart tail")) ||
-      (st = hip_check(hipMemsetAsync(tp.prod.as<uint32_t>() + nprod, 0, kWaveProducts * 4, s), "memset prod tail")))
-    return st;
-  hipLaunchKernelGGL((k_chunk_prods<true>), dim3(grid1(std::max(nch, 1), 256)), dim3(256), 0, s, nch,
-                     d_centry.as<int32_t>(), d_ctile.as<int32_t>(), d_emask.as<uint32_t>(), d_ecoff.as<int32_t>(),
-                     d_owner.as<uint8_t>(), (int32_t)ns2, nullptr, d_pbase.as<int64_t>(), tp.pstart.as<int64_t>(),
-                     tp.pcnt.as<uint64_t>(), tp.prod.as<uint32_t>());
+  // The dense kernel reads the entries themselves.
+  tp.chunk_entry = std::move(d_centry);
+  tp.entry_mask = std::move(d_emask);
+  tp.entry_coff = std::move(d_ecoff);
+  tp.n_prod = n;
   if ((st = hip_check(hipGetLastError(), "tile builder launch"))) return st;
-  st = hip_check(hipStreamSynchronize(s), "tile build");
-  pt.mark("  tiles: product lists");
-  return st;
+  return hip_check(hipStreamSynchronize(s), "tile build");
 }
 
 int launch_tile_products(const TilePlan &tp, bool q_trans, const double *P, const double *Q, double *O,
                          hipStream_t s) {
   if (tp.n_tiles == 0) return CQMM_OK;
-  return launch_any(0, q_trans, tile_kind(tp), tile_launch_args(tp, P, Q, O), tp.n_tiles, tp.wgs, s);
+  return launch_tile_args(tp, q_trans, 0, tile_launch_args(tp, P, Q, O), s);
 }
 
 // Mixed block sizes: the uniform builder's steps with element offsets and

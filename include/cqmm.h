@@ -39,8 +39,9 @@ extern "C" {
 #define CQMM_FP32 2u         /* run the block products in FP32 (MFMA, FP32 accumulate) */
 #define CQMM_NO_SYNC 4u      /* return without synchronising the plan stream */
 #define CQMM_FP32_ACC64 8u   /* with CQMM_FP32: sum each block's products in FP64 */
-#define CQMM_FP32_RUN64 16u  /* with CQMM_FP32: sum a block's products within one chunk of the
-                                tile schedule (at most 15) in FP32, the chunks in FP64 */
+#define CQMM_FP32_RUN64 16u  /* with CQMM_FP32: a kernel may sum up to 15 consecutive products of
+                                a block in FP32 before adding them in FP64 (every kernel here
+                                adds each product in FP64, as CQMM_FP32_ACC64) */
 #define CQMM_BF16X3 32u      /* with CQMM_FP32: split-BF16 x3 products (each operand split into
                                 two BF16 halves, hi.hi + hi.lo + lo.hi in BF16 MFMA with FP32
                                 accumulation per block product, FP64 block sums); needs a tile
