@@ -78,14 +78,14 @@ struct TilePlan {
   DevBuf prod;         // uint32 [n_prod+64] LDS element offsets of the two operands (left | right << 16)
   DevBuf tile_out;     // int32 [n_tiles*64] output block of slot row*8+col, or -1
   DevBuf wave_out;     // int32 [n_tiles*4*16] output block of (tile, wavefront, slot), or -1
-  // Uniform 9, 13, 16 (k_wave_products): the 4x4-block quadrants of the tiles
-  // that hold an output block, each the work of one wavefront. wave_out is then
-  // [n_wave*16], pstart [n_wave+1] the first record word of each quadrant and
-  // prod the record words (64 words of padding).
+  // Uniform sizes (k_wave_products; 4x4 blocks, dense: k_quad4): the 4x4-block
+  // quadrants of the tiles that hold an output block, each the work of one
+  // wavefront. wave_out is then [n_wave*16] (row * 4 + column within the
+  // quadrant), pstart [n_wave+1] the first record word of each quadrant and prod
+  // the record words, with padding.
   int32_t n_wave = 0;
-  // 4x4 blocks (dense): each wavefront computes a 4x4-block quadrant of the
-  // tile per entry with one MFMA; no product lists. wave_out then holds the
-  // quadrant's blocks (row * 4 + column within the quadrant).
+  // Mixed sizes up to 4x4 (dense): each wavefront computes a 4x4-block quadrant
+  // of the tile per entry with one MFMA; no product lists.
   bool dense = false;
   bool quad = false;   // class tiles (k_tile_quad): one row and one column block size per tile
   int32_t wgs = 0;     // class tiles: workgroups of a persistent launch (0: one per tile)

@@ -12,8 +12,9 @@
 //  * an entry of a tile is one contraction atom x with its (up to 8) left
 //    operand blocks P(row, x) and (up to 8) right operand blocks Q(column, x);
 //    entries of a tile are in ascending x (type 1: the reference's k order);
-//  * uniform 9, 13, 16: each 4x4-block quadrant of a tile is the work of one
-//    wavefront of its own, driven by a list of records (k_wave_products);
+//  * uniform sizes: each 4x4-block quadrant of a tile is the work of one
+//    wavefront of its own, driven by a list of records (k_wave_products,
+//    k_quad4);
 //  * the other kernels run a tile with one workgroup (4 wavefronts, three
 //    workgroups per CU). Chunks of entries have their operand blocks copied
 //    HBM->LDS (global_load_lds, no registers) into one of two stages while the
@@ -82,23 +83,10 @@ __device__ inline s16x4 half_of(const float *k, int i) {
   return __builtin_bit_cast(s16x4, (uint64_t)__float_as_uint(k[i]) | ((uint64_t)__float_as_uint(k[i + 1]) << 32));
 }
 
-// Lane N of each row of 16 lanes, for all lanes of that row.
-template <int N>
-__device__ inline float row_bcast(float x) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + N, 0xf, 0xf, true));
-}
-template <int N>
-__device__ inline double row_bcast(double x) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x150 + N, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x150 + N, 0xf, 0xf, true);
-  return __hiloint2double(hi, lo);
-}
-
 constexpr int kWaves = 4;                    // wavefronts per workgroup (one tile)
 constexpr int kTileThreads = 64 * kWaves;
 constexpr int kSlots = 64 / kWaves;          // output blocks per wavefront
 static_assert(8 % kWaves == 0, "a tile row of 8 blocks is split evenly over the wavefronts");
-constexpr int kStageBytes = 24 * 1024;       // one of the two operand stages (three workgroups per CU)
 // LDS reads of a block product never mask rows or columns beyond NSF: those
 // lanes only feed accumulator rows/columns >= NSF, which are never written.
 // Only the contraction index 4*s+g >= NSF at the last k-step is zeroed (both
@@ -110,26 +98,10 @@ constexpr int kWaveProducts = 64;            // products per wavefront per chunk
 constexpr int kDenseNsf = 4;                 // block size of the dense-quadrant kernel
 constexpr int kDenseEntries = 64;            // entries per chunk at most there (one per lane)
 
-// Operand blocks per chunk (FP64 sizing): what fits kStageBytes, but at
-// least the 16 blocks one entry can bring (8 left + 8 right), so every entry
-// fits a stage on its own (16x16 blocks: 32 KB stages, two workgroups per CU).
-constexpr int stage_cap(int nsf) {
-  return kStageBytes / (nsf * nsf * 8) > 16 ? kStageBytes / (nsf * nsf * 8) : 16;
-}
-
-int tile_cap(int nsf) { return stage_cap(nsf); }
-
 // Prefetch loads are unconditional (indices clamped or arrays padded) so that
 // no value is consumed before the next barrier: a use right after the load
 // would make the wavefront wait for every outstanding load, including the
 // stage copies that are meant to overlap the compute.
-//
-// Operand list of a chunk with nb > 0 blocks: lane k holds the operand of
-// block min(w + kWaves*k, nb - 1) (lanes past wavefront w's blocks are unused).
-__device__ inline int32_t load_chunk_list(const int32_t *__restrict__ list, int64_t lbeg, int32_t nb, int w,
-                                          int lane) {
-  return list[lbeg + min(w + kWaves * lane, nb - 1)];
-}
 
 // One 256-byte piece of a block copy: lane l moves dword OFF/4 + l. The
 // immediate offset applies to both the global and the LDS address (one M0 per
@@ -138,34 +110,6 @@ template <int OFF>
 __device__ inline void dma_piece(const uint32_t *src, uint32_t *dst) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
                                    (__attribute__((address_space(3))) void *)dst, 4, OFF, 0);
-}
-
-template <int... I>
-__device__ inline void dma_full_pieces(const uint32_t *src, uint32_t *dst, std::integer_sequence<int, I...>) {
-  (dma_piece<I * 256>(src, dst), ...);
-}
-
-// Issue the HBM->LDS copies of a chunk's operand blocks without waiting:
-// wavefront w copies blocks w, w+kWaves, ... (operands in lv) with
-// global_load_lds_dword; lane l moves dword k*64+l of a block to
-// stage + block*DW + k*64 + l.
-template <int NSF, class T>
-__device__ inline void issue_stage(int32_t lv, int32_t nb, const T *__restrict__ P, const T *__restrict__ Q,
-                                   T *stage, int w, int lane) {
-  constexpr int NS2 = NSF * NSF;
-  constexpr int DW = NS2 * (int)sizeof(T) / 4;
-  constexpr int NF = DW / 64;          // full 64-dword pieces
-  constexpr int TAIL = DW - 64 * NF;   // dwords of the last piece
-  const int32_t nbw = nb > w ? (nb - w + kWaves - 1) / kWaves : 0;
-  for (int32_t k = 0; k < nbw; ++k) {
-    const int32_t lb = __builtin_amdgcn_readlane(lv, k);
-    const uint32_t *src = (const uint32_t *)((lb < 0 ? Q : P) + (int64_t)(lb & 0x7fffffff) * NS2) + lane;
-    uint32_t *dst = (uint32_t *)(stage + (w + kWaves * k) * NS2);
-    dma_full_pieces(src, dst, std::make_integer_sequence<int, NF>{});
-    if constexpr (TAIL > 0) {
-      if (lane < TAIL) dma_piece<NF * 256>(src, dst);
-    }
-  }
 }
 
 using cq::TileArgs;
@@ -273,6 +217,7 @@ struct FragOff {
 // Ring of operand blocks of a wavefront: what its share of the 160 KB LDS
 // holds beside the record words, with 2 wavefronts per SIMD (FP64) or 3.
 constexpr int kWaveWords = 256;  // record words in LDS
+constexpr int kWavePad = 128;    // words after a plan's last record
 constexpr int wave_per_simd(int mode) { return mode == 0 ? 2 : 3; }
 constexpr int wave_dmas(int nsf, int size) { return (nsf * nsf * size + 1023) / 1024; }  // copies per block
 constexpr int wave_ring(int mode, int nsf) {
@@ -520,127 +465,104 @@ k_wave_products(const ARG arg) {
   }
 }
 
-// 4x4 blocks: a tile is 32x32 elements, and wavefront w owns its 16x16
-// quadrant (block rows 4*(w/2)..+3, block columns 4*(w%2)..+3). One
-// 16x16x4 MFMA per entry covers the entry's whole contraction (4) for all 16
-// blocks of the quadrant at once: lane (r, g) supplies P(row 4*(w/2)+r/4,
-// x)[r%4][g] and Q(column 4*(w%2)+r/4, x)[g][r%4], zero where the entry has no
-// such block. A block pair whose output block does not exist only feeds
-// accumulator elements that are never written; every output block sums its
-// products in entry (x) order, one fused step per product, as the triplet
-// kernel does. Chunk c's copies are waited for (one barrier), chunk c+1's issued
-// into the other stage, then chunk c computed; the chunk's entries are at most
-// 64, one per lane.
+// 4x4 blocks: one wavefront computes 4x4 output blocks (a quadrant of a tile), on
+// its own. A record (contraction atom) is eight block indices, four rows and
+// four columns, -1 where the block does not exist. One matrix step covers the
+// record's whole contraction (4) for all 16 blocks at once: lane (r, g) supplies
+// left row r/4, element [r%4][g], and right column r/4, element [g][r%4]. A block pair
+// whose output block does not exist only feeds accumulator elements that are
+// never written; every output block sums its products in ascending
+// contraction atom, one fused step per product, as the triplet kernel does.
+//
+// A record's blocks are copied memory -> LDS by one instruction (16 bytes a
+// lane, absent blocks from a block of zeros), three records ahead. FP64: in LDS
+// the halves (type 1 right operands: the 16-byte pairs) of blocks 2 and 3 of
+// the rows and of the columns are swapped, so that the operand reads have no
+// bank conflict.
+//
+// What bounds it: a record takes one 72-cycle f64 matrix step and about ten VALU
+// instructions, and copies from L2 (13 to 16 TB/s) what its products read: 512
+// atoms, 2.0e7 products, 0.215 ms. One workgroup per 8x8 tile with a barrier per
+// chunk took 0.80 ms; a list of products per output block with v_mfma_f64_4x4x4
+// (four output blocks to a wavefront) 0.45 ms, as it copies 2 blocks per product
+// and not the 0.6 to 0.9 of a record. One McWeeny batch of 4 x 64 atoms
+// 73.7 -> 26.9 ms.
+__device__ __attribute__((aligned(128))) uint32_t g_zero_block[32];
+
 template <int MODE, bool QT, class ARG>
-__global__ void __launch_bounds__(kTileThreads) k_tile_dense4(
-    const ARG arg) {
+__global__ void __launch_bounds__(64) k_quad4(const ARG arg) {
   using T = typename std::conditional<MODE == 0, double, float>::type;
-  constexpr int NS2 = kDenseNsf * kDenseNsf;
-  constexpr int STAGE = stage_cap(kDenseNsf) * NS2 + kLdsPad * (int)(8 / sizeof(T));
-  __shared__ T stage0[STAGE];
-  __shared__ T stage1[STAGE];
+  constexpr int BYTES = 16 * (int)sizeof(T), LPB = BYTES / 16, SLOT = 8 * BYTES, AHEAD = 3;
+  __shared__ __attribute__((aligned(256))) char lds[(AHEAD + 1) * SLOT];
   TileArgs a;
   const int32_t tile = tile_select(arg, a);
-  if (tile < 0) return;  // the whole workgroup leaves together
-  const int32_t *__restrict__ tile_chunk = a.tile_chunk;
-  const int64_t *__restrict__ chunk_lbeg = a.chunk_lbeg;
-  const int32_t *__restrict__ list = a.list;
-  const int32_t *__restrict__ chunk_entry = a.chunk_entry;
-  const uint32_t *__restrict__ emask = a.emask;
-  const int32_t *__restrict__ ecoff = a.ecoff;
-  const int32_t *__restrict__ wave_out = a.wave_out;
-  const T *__restrict__ P = static_cast<const T *>(a.P);
-  const T *__restrict__ Q = static_cast<const T *>(a.Q);
+  if (tile < 0) return;
+  const int lane = threadIdx.x, r = lane & 15, g = lane >> 4;
   T *__restrict__ O = static_cast<T *>(a.O);
-  const int tid = threadIdx.x;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63, r = lane & 15, g = lane >> 4;
-  const int qr = w >> 1, qc = w & 1;
-  const int ua = 4 * qr + (r >> 2);  // tile row of this lane's left operand
-  const int cb = 4 * qc + (r >> 2);  // tile column of this lane's right operand
-  const int oa = (r & 3) + 4 * g;    // P(row, x)[r % 4][g]
-  const int ob = QT ? (r & 3) + 4 * g : g + 4 * (r & 3);  // Q[g][r % 4]
-  const uint32_t below_a = (1u << ua) - 1u, below_b = (1u << cb) - 1u;
-  const uint32_t quad_rows = 0xfu << (4 * qr), quad_cols = 0xfu << (8 + 4 * qc);
   dbl4 a64 = {0.0, 0.0, 0.0, 0.0};
   flt4 a32 = {0.f, 0.f, 0.f, 0.f};
-  const int32_t c0 = tile_chunk[tile], c1 = tile_chunk[tile + 1];
-  if (c0 < c1) {
-    // Per-chunk operand-list and entry bounds of the tile in registers, 64
-    // chunks at a time (lane l: chunk wb + l, clamped to c1).
-    int32_t wb = c0;
-    int32_t cc = min(wb + lane, c1);
-    int64_t wcl = chunk_lbeg[cc];
-    int32_t wce = chunk_entry[cc];
-    auto cl_at = [&](int32_t x) { return readlane64(wcl, min(x, c1) - wb); };
-    auto ce_at = [&](int32_t x) { return __builtin_amdgcn_readlane(wce, min(x, c1) - wb); };
-    // The entries of a chunk, lane i = entry i (index clamped to the chunk).
-    auto entry_regs = [&](int32_t e0, int32_t e1, uint32_t &m, int32_t &o) {
-      const int32_t e = min(e0 + lane, e1 - 1);
-      m = emask[e];
-      o = ecoff[e];
+  const int64_t w0 = a.pstart[tile];
+  const int32_t n = (int32_t)((a.pstart[tile + 1] - w0) >> 3);
+  if (n > 0) {
+    // Copy lanes: LPB lanes for each of the record's blocks.
+    const int blk = lane / LPB, piece = lane % LPB;
+    const int swap = MODE == 0 && (blk & 2) ? (blk < 4 || QT ? 4 : 1) : 0;
+    const char *base = static_cast<const char *>(blk < 4 ? a.P : a.Q) + 16 * (piece ^ swap);
+    const char *zero = (const char *)g_zero_block + 16 * piece;
+    auto copy = [&](uint32_t words, int i, int slot) {
+      const uint32_t x = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * (8 * i + (blk & 7)), (int)words);
+      const char *src = x == ~0u ? zero : base + (uint64_t)x * BYTES;
+      if (LPB == 8 || lane < 8 * LPB)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
+                                         (__attribute__((address_space(3))) void *)(lds + slot * SLOT), 16, 0, 0);
     };
-    uint32_t em, emn = 0;
-    int32_t eo, eon = 0;
-    int32_t lvn = 0;
-    {
-      const int64_t cl0 = cl_at(c0), cl1 = cl_at(c0 + 1);
-      const int32_t lv0 = load_chunk_list(list, cl0, (int32_t)(cl1 - cl0), w, lane);
-      issue_stage<kDenseNsf, T>(lv0, (int32_t)(cl1 - cl0), P, Q, stage0, w, lane);
-      entry_regs(ce_at(c0), ce_at(c0 + 1), emn, eon);
-      if (c0 + 1 < c1) lvn = load_chunk_list(list, cl1, (int32_t)(cl_at(c0 + 2) - cl1), w, lane);
-    }
-    for (int32_t c = c0; c < c1; ++c) {
-      __builtin_amdgcn_s_waitcnt(0);
-      __syncthreads();
-      const bool odd = ((c - c0) & 1) != 0;
-      const T *cur = odd ? stage1 : stage0;
-      em = emn;
-      eo = eon;
-      const int32_t ne = ce_at(c + 1) - ce_at(c);
-      if (c + 1 < c1) {
-        const int64_t cl1 = cl_at(c + 1), cl2 = cl_at(c + 2);
-        issue_stage<kDenseNsf, T>(lvn, (int32_t)(cl2 - cl1), P, Q, odd ? stage0 : stage1, w, lane);
-        entry_regs(ce_at(c + 1), ce_at(c + 2), emn, eon);
-        if (c + 2 < c1) lvn = load_chunk_list(list, cl2, (int32_t)(cl_at(c + 3) - cl2), w, lane);
-      }
-      for (int i = 0; i < ne; ++i) {
-        const uint32_t m = (uint32_t)__builtin_amdgcn_readlane((int)em, i);
-        if ((m & quad_rows) == 0 || (m & quad_cols) == 0) continue;  // no block pair in this quadrant
-        const int32_t base = __builtin_amdgcn_readlane(eo, i);
-        const uint32_t ym = m & 0xffu, bm = (m >> 8) & 0xffu;
-        const int ia = base + __popc(ym & below_a);
-        const int ib = base + __popc(ym) + __popc(bm & below_b);
-        T a = cur[ia * NS2 + oa], b = cur[ib * NS2 + ob];
-        if (((ym >> ua) & 1u) == 0) a = (T)0;
-        if (((bm >> cb) & 1u) == 0) b = (T)0;
+    // Operand lanes: byte offset of the lane's element in a record's stage.
+    const int u = r >> 2, m = r & 3;
+    const int fa = BYTES * u + ((int)sizeof(T) * (m + 4 * g) ^ (MODE == 0 && (u & 2) ? 64 : 0));
+    const int fb = BYTES * (4 + u) + (QT ? (int)sizeof(T) * (m + 4 * g) ^ (MODE == 0 && (u & 2) ? 64 : 0)
+                                         : (int)sizeof(T) * (g + 4 * m) ^ (MODE == 0 && (u & 2) ? 16 : 0));
+    // The words of 8 records, one per lane, and of the 8 after them. The copies
+    // and words past the quadrant's last record are those of the next quadrant
+    // (or the list's 16 records of padding), never used.
+    const uint32_t *words = a.prod + w0 + lane;
+    uint32_t w = words[0];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) copy(w, i, i);
+    for (int32_t rec = 0; rec < n; rec += 8) {
+      const uint32_t wn = words[8 * (int64_t)(rec + 8)];
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (rec + i >= n) break;
+        copy(i + AHEAD < 8 ? w : wn, (i + AHEAD) & 7, (i + AHEAD) & 3);
+        asm volatile("" ::: "memory");
+        // The record's copy is older than AHEAD others and, at first, the load of wn.
+        if (i < AHEAD) __builtin_amdgcn_s_waitcnt((AHEAD + 1) | 0xf70);
+        else __builtin_amdgcn_s_waitcnt(AHEAD | 0xf70);
+        asm volatile("" ::: "memory");
+        const T x = *(const T *)(lds + (i & 3) * SLOT + fa), y = *(const T *)(lds + (i & 3) * SLOT + fb);
         if constexpr (MODE == 0) {
-          a64 = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, a64, 0, 0, 0);
+          a64 = __builtin_amdgcn_mfma_f64_16x16x4f64(x, y, a64, 0, 0, 0);
         } else if constexpr (MODE == 1) {
-          a32 = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, a32, 0, 0, 0);
+          a32 = __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, a32, 0, 0, 0);
         } else {
-          const flt4 t = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, flt4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+          const flt4 t = __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, flt4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
           for (int e = 0; e < 4; ++e) a64[e] += (double)t[e];
         }
       }
-      if (c + 4 > wb + 63 && c + 1 < c1) {  // next iteration reads up to chunk c + 3
-        wb = c + 1;
-        cc = min(wb + lane, c1);
-        wcl = chunk_lbeg[cc];
-        wce = chunk_entry[cc];
-      }
+      w = wn;
     }
+    __builtin_amdgcn_s_waitcnt(0xf70);  // no copy into LDS outlives the wavefront
   }
   // FP64 accumulator D[g+4e][r], FP32 D[4g+e][r]: quadrant row R, column r is
   // element (R % 4, r % 4) of block (R / 4, r / 4).
-  const int32_t *wo = wave_out + ((int64_t)tile * kWaves + w) * 16;
+  const int32_t *wo = a.wave_out + (int64_t)tile * 16;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int rq = MODE == 0 ? e : g, ri = MODE == 0 ? g : e;
-    const int32_t blk = wo[rq * 4 + (r >> 2)];
-    if (blk >= 0)
-      O[(int64_t)blk * NS2 + ri + 4 * (r & 3)] = MODE == 1 ? (T)a32[e] : (T)a64[e];
+    const int32_t o = wo[rq * 4 + (r >> 2)];
+    if (o >= 0) O[(int64_t)o * 16 + ri + 4 * (r & 3)] = MODE == 1 ? (T)a32[e] : (T)a64[e];
   }
 }
 
@@ -657,15 +579,6 @@ __global__ void k_chunk_lbeg(const int32_t *__restrict__ chunk_entry, const int6
                              int64_t nc1, int64_t *__restrict__ out) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c < nc1) out[c] = entry_lbeg[chunk_entry[c]];
-}
-
-// Operand-list start of each entry relative to its chunk's first operand.
-__global__ void k_entry_coff(const int32_t *__restrict__ chunk_entry, const int64_t *__restrict__ entry_lbeg,
-                             int64_t nc, int32_t *__restrict__ coff) {
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= nc) return;
-  const int64_t base = entry_lbeg[chunk_entry[c]];
-  for (int32_t e = chunk_entry[c]; e < chunk_entry[c + 1]; ++e) coff[e] = (int32_t)(entry_lbeg[e] - base);
 }
 
 __global__ void k_iota32(int32_t *__restrict__ v, int64_t n) {
@@ -703,31 +616,6 @@ __global__ void k_entry_fill(const uint64_t *__restrict__ key, const int32_t *__
   if (pos == 0 || eid[pos - 1] != eid[pos]) etile[e] = (int32_t)(key[pos] / (uint64_t)nx);
 }
 
-__global__ void k_entry_mask(const int32_t *__restrict__ ep, const int32_t *__restrict__ eq, int64_t ne,
-                             uint32_t *__restrict__ mask, int64_t *__restrict__ cnt) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= ne) return;
-  uint32_t m = 0;
-  for (int u = 0; u < 8; ++u) {
-    if (ep[e * 8 + u] >= 0) m |= 1u << u;
-    if (eq[e * 8 + u] >= 0) m |= 1u << (8 + u);
-  }
-  mask[e] = m;
-  cnt[e] = __popc(m);
-}
-
-// Operand list of each entry: present left blocks by row, then right blocks by column.
-__global__ void k_list_fill(const int32_t *__restrict__ ep, const int32_t *__restrict__ eq,
-                            const int64_t *__restrict__ lbeg, int64_t ne, int32_t *__restrict__ list) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= ne) return;
-  int64_t o = lbeg[e];
-  for (int u = 0; u < 8; ++u)
-    if (ep[e * 8 + u] >= 0) list[o++] = ep[e * 8 + u];
-  for (int u = 0; u < 8; ++u)
-    if (eq[e * 8 + u] >= 0) list[o++] = (int32_t)((uint32_t)eq[e * 8 + u] | 0x80000000u);
-}
-
 // tebeg[t] = first entry of tile t (entries are sorted by tile), t = 0..n_tiles.
 __global__ void k_tile_ebeg(const int32_t *__restrict__ etile, int64_t ne, int32_t n_tiles,
                             int32_t *__restrict__ tebeg) {
@@ -757,30 +645,6 @@ __device__ inline void entry_wave_counts(uint32_t m, const uint8_t *__restrict__
   }
 }
 
-// Chunks of a tile: at most max_entries consecutive entries whose operand
-// blocks fit `cap`. With FILL unset, counts them; with FILL set, writes each
-// chunk's first entry.
-template <bool FILL>
-__global__ void k_chunks(const int32_t *__restrict__ tebeg, const uint32_t *__restrict__ mask, int32_t n_tiles,
-                         int32_t cap, int32_t max_entries, const int32_t *__restrict__ tchunk,
-                         int32_t *__restrict__ out) {
-  const int32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n_tiles) return;
-  int32_t nch = 0, sum = 0, ne = 0;
-  for (int32_t e = tebeg[t]; e < tebeg[t + 1]; ++e) {
-    const int32_t c = __popc(mask[e]);
-    if (nch == 0 || sum + c > cap || ne == max_entries) {
-      if (FILL) out[tchunk[t] + nch] = e;
-      ++nch;
-      sum = 0;
-      ne = 0;
-    }
-    sum += c;
-    ++ne;
-  }
-  if (!FILL) out[t] = nch;
-}
-
 // Tile of each chunk.
 __global__ void k_chunk_tile(const int32_t *__restrict__ tchunk, int32_t n_tiles, int32_t *__restrict__ ctile) {
   const int32_t t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -788,15 +652,15 @@ __global__ void k_chunk_tile(const int32_t *__restrict__ tchunk, int32_t n_tiles
   for (int32_t c = tchunk[t]; c < tchunk[t + 1]; ++c) ctile[c] = t;
 }
 
-// Records of k_wave_products, one wavefront per quadrant q (src[q] = tile * 4 +
-// quadrant): of the tile's entries (ascending contraction atom) those with a
-// product in the quadrant; the rows and columns that have one, then their
-// block indices. A record holds at most `cap` blocks: an entry with more
-// becomes several records over the same columns, each with some of its rows
-// (cap >= 5). Count pass (FILL unset): words, products and blocks of each quadrant.
-template <bool FILL>
+// Records of the quadrant kernels, one wavefront per quadrant q (src[q] =
+// tile * 4 + quadrant): of the tile's entries (ascending contraction atom) those
+// with a product in the quadrant. k_wave_products (QUAD4 unset): rows and
+// columns that have one, then their block indices. k_quad4: eight block indices,
+// -1 for the rows and columns without. Count pass (FILL unset): words, products
+// and blocks of each quadrant.
+template <bool FILL, bool QUAD4>
 __global__ void __launch_bounds__(256) k_wave_records(
-    const int32_t *__restrict__ src, int32_t n_wave, int32_t cap, const int32_t *__restrict__ wave_out,
+    const int32_t *__restrict__ src, int32_t n_wave, const int32_t *__restrict__ wave_out,
     const int32_t *__restrict__ tebeg, const int32_t *__restrict__ ep, const int32_t *__restrict__ eq,
     int64_t *__restrict__ nword, int64_t *__restrict__ nprod, int64_t *__restrict__ nload,
     const int64_t *__restrict__ beg, uint32_t *__restrict__ out) {
@@ -828,40 +692,24 @@ __global__ void __launch_bounds__(256) k_wave_records(
         rows |= (uint32_t)(c != 0) << k;
       }
     }
-    // The entry's rows in `parts` records of nearly equal size.
-    const int nr = __popc(rows), nc = __popc(cols);
-    const int per = cap - nc, parts = nr == 0 ? 0 : (nr + per - 1) / per;
-    const int len = parts * (1 + nc) + nr;
+    const int nb = __popc(rows) + __popc(cols), len = rows == 0 ? 0 : QUAD4 ? 8 : 1 + nb;
     int before = len;  // inclusive prefix sum of the records' words over the lanes
     for (int off = 1; off < 64; off <<= 1) {
       const int v = __shfl_up(before, off, 64);
       if (lane >= off) before += v;
     }
-    if (FILL && parts > 0) {
+    if (FILL && rows != 0) {
       int64_t o = at + before - len;
-      int done = 0;
-      for (int part = 0; part < parts; ++part) {
-        const int take = (nr - done + parts - part - 1) / (parts - part);
-        const int64_t head = o++;
-        uint32_t rm = 0;
-        int seen = 0;
-        for (int k = 0; k < 4; ++k)
-          if (rows >> k & 1u) {
-            if (seen >= done && seen < done + take) {
-              rm |= 1u << k;
-              out[o++] = (uint32_t)b[k];
-            }
-            ++seen;
-          }
-        for (int k = 0; k < 4; ++k)
-          if (cols >> k & 1u) out[o++] = (uint32_t)b[4 + k];
-        out[head] = rm | cols << 4;
-        done += take;
+      const uint32_t here = rows | cols << 4;
+      if (!QUAD4) out[o++] = here;
+      for (int k = 0; k < 8; ++k) {
+        if (here >> k & 1u) out[o++] = (uint32_t)b[k];
+        else if (QUAD4) out[o++] = ~0u;
       }
     }
     at += __shfl(before, 63, 64);
     prods += np;
-    loads += nr + parts * nc;
+    loads += nb;
   }
   if (!FILL) {
     for (int off = 32; off > 0; off >>= 1) {
@@ -1748,7 +1596,7 @@ int launch_kind(int kind, const ARG &arg, int32_t n, int32_t wgs, hipStream_t s)
     gridx = std::min(gridx, 8u * (unsigned)((wgs + 7) / 8));
   const dim3 blk(kTileThreads);
   switch (kind) {
-    case kKindDense4: hipLaunchKernelGGL((k_tile_dense4<MODE, QT, ARG>), dim3(gridx), blk, 0, s, arg); break;
+    case kKindDense4: hipLaunchKernelGGL((k_quad4<MODE, QT, ARG>), dim3(gridx), dim3(64), 0, s, arg); break;
     case kKindDenseMx: hipLaunchKernelGGL((k_tile_dense_mx<MODE, QT, ARG>), dim3(gridx), blk, 0, s, arg); break;
     case kKindMixedSmall: hipLaunchKernelGGL((k_tile_mixed<MODE, QT, kStgSmall, ARG>), dim3(gridx), blk, 0, s, arg); break;
     case kKindMixedLarge: hipLaunchKernelGGL((k_tile_mixed<MODE, QT, kStgLarge, ARG>), dim3(gridx), blk, 0, s, arg); break;
@@ -2053,7 +1901,6 @@ int build_tiles(const TileBuildInput &in, TilePlan &tp, hipStream_t s) {
   cq::PhaseTimer pt;
   const int64_t n = in.n_trip;
   const int64_t ns2 = (int64_t)in.nsf * in.nsf;
-  const int32_t cap = tile_cap(in.nsf);
   int st;
   tp = TilePlan();
   tp.nsf = in.nsf;
@@ -2078,20 +1925,18 @@ int build_tiles(const TileBuildInput &in, TilePlan &tp, hipStream_t s) {
         for (int c = 0; c < 8; ++c)
           wave_out[(t * kWaves + (u >> 2) * 2 + (c >> 2)) * 16 + (u & 3) * 4 + (c & 3)] = tout32[t * 64 + u * 8 + c];
   });
-  if (!tp.dense) {
-    // Only the quadrants with output blocks are work.
-    src.reserve((size_t)in.n_tiles * kWaves);
-    for (int64_t q = 0; q < (int64_t)in.n_tiles * kWaves; ++q) {
-      bool any = false;
-      for (int k = 0; k < 16; ++k) any |= wave_out[q * 16 + k] >= 0;
-      if (!any) continue;
-      if ((int64_t)src.size() != q)
-        for (int k = 0; k < 16; ++k) wave_out[src.size() * 16 + k] = wave_out[q * 16 + k];
-      src.push_back((int32_t)q);
-    }
-    wave_out.resize(src.size() * 16);
-    tp.n_wave = (int32_t)src.size();
+  // Only the quadrants with output blocks are work.
+  src.reserve((size_t)in.n_tiles * kWaves);
+  for (int64_t q = 0; q < (int64_t)in.n_tiles * kWaves; ++q) {
+    bool any = false;
+    for (int k = 0; k < 16; ++k) any |= wave_out[q * 16 + k] >= 0;
+    if (!any) continue;
+    if ((int64_t)src.size() != q)
+      for (int k = 0; k < 16; ++k) wave_out[src.size() * 16 + k] = wave_out[q * 16 + k];
+    src.push_back((int32_t)q);
   }
+  wave_out.resize(src.size() * 16);
+  tp.n_wave = (int32_t)src.size();
   if ((st = tp.wave_out.alloc(wave_out.size() * 4))) return st;
   if ((st = hip_check(hipMemcpyAsync(tp.wave_out.p, wave_out.data(), wave_out.size() * 4, hipMemcpyHostToDevice, s),
                       "H2D wave_out")) ||
@@ -2129,9 +1974,9 @@ int build_tiles(const TileBuildInput &in, TilePlan &tp, hipStream_t s) {
     return st;
   const int64_t ne = ne32;
   tp.n_entries = ne;
-  DevBuf d_ep, d_eq, d_etile, d_cnt, d_emask, d_elbeg, d_ecoff;
+  DevBuf d_ep, d_eq, d_etile, d_tebeg;
   if ((st = d_ep.alloc(ne * 8 * 4)) || (st = d_eq.alloc(ne * 8 * 4)) || (st = d_etile.alloc(ne * 4)) ||
-      (st = d_cnt.alloc(ne * 8)))
+      (st = d_tebeg.alloc(((size_t)in.n_tiles + 1) * 4)))
     return st;
   hipLaunchKernelGGL(k_fill_i32, dim3(grid1(ne * 8, 256)), dim3(256), 0, s, d_ep.as<int32_t>(), ne * 8, -1);
   hipLaunchKernelGGL(k_fill_i32, dim3(grid1(ne * 8, 256)), dim3(256), 0, s, d_eq.as<int32_t>(), ne * 8, -1);
@@ -2141,95 +1986,44 @@ int build_tiles(const TileBuildInput &in, TilePlan &tp, hipStream_t s) {
   d_eid.release();
   d_perm2.release();
   d_key2.release();
-  if ((st = d_emask.alloc(ne * 4)) || (st = d_elbeg.alloc((ne + 1) * 8))) return st;
-  hipLaunchKernelGGL(k_entry_mask, dim3(grid1(ne, 256)), dim3(256), 0, s, d_ep.as<int32_t>(), d_eq.as<int32_t>(), ne,
-                     d_emask.as<uint32_t>(), d_cnt.as<int64_t>());
-  if ((st = hip_check(hipMemsetAsync(d_elbeg.p, 0, 8, s), "memset lbeg"))) return st;
-  if ((st = inclusive_scan(d_cnt.as<int64_t>(), d_elbeg.as<int64_t>() + 1, (size_t)ne, s))) return st;
-  int64_t nl = 0;
-  if ((st = hip_check(hipMemcpyAsync(&nl, d_elbeg.as<int64_t>() + ne, 8, hipMemcpyDeviceToHost, s), "D2H loads")) ||
-      (st = hip_check(hipStreamSynchronize(s), "load count")))
-    return st;
-  tp.n_loads = nl;
-  DevBuf d_tebeg, d_nch;
-  if ((st = d_tebeg.alloc(((size_t)in.n_tiles + 1) * 4)) || (st = d_nch.alloc((size_t)in.n_tiles * 4))) return st;
   hipLaunchKernelGGL(k_tile_ebeg, dim3(grid1((int64_t)in.n_tiles + 1, 256)), dim3(256), 0, s, d_etile.as<int32_t>(), ne,
                      in.n_tiles, d_tebeg.as<int32_t>());
-  if (!tp.dense) {
-    // Entry records of the quadrants: count, first record of each, fill.
-    const size_t nq = src.size();
-    DevBuf d_src, d_nrec, d_nprod, d_nload;
-    if ((st = d_src.alloc(nq * 4)) || (st = d_nrec.alloc(nq * 8)) || (st = d_nprod.alloc(nq * 8)) ||
-        (st = d_nload.alloc(nq * 8)) || (st = tp.pstart.alloc((nq + 1) * 8)))
-      return st;
-    if ((st = hip_check(hipMemcpyAsync(d_src.p, src.data(), nq * 4, hipMemcpyHostToDevice, s), "H2D quadrants"))) return st;
-    const dim3 grid(grid1((int64_t)nq, 4));
-    hipLaunchKernelGGL((k_wave_records<false>), grid, dim3(256), 0, s, d_src.as<int32_t>(), tp.n_wave,
-                       8, tp.wave_out.as<int32_t>(), d_tebeg.as<int32_t>(), d_ep.as<int32_t>(), d_eq.as<int32_t>(),
-                       d_nrec.as<int64_t>(), d_nprod.as<int64_t>(), d_nload.as<int64_t>(), nullptr, nullptr);
-    int64_t nrec = 0, nprod = 0, nload = 0;
-    if ((st = hip_check(hipMemsetAsync(tp.pstart.p, 0, 8, s), "memset pstart")) ||
-        (st = inclusive_scan(d_nrec.as<int64_t>(), tp.pstart.as<int64_t>() + 1, nq, s)) ||
-        (st = inclusive_scan(d_nprod.as<int64_t>(), d_nprod.as<int64_t>(), nq, s)) ||
-        (st = inclusive_scan(d_nload.as<int64_t>(), d_nload.as<int64_t>(), nq, s)) ||
-        (st = hip_check(hipMemcpyAsync(&nrec, tp.pstart.as<int64_t>() + nq, 8, hipMemcpyDeviceToHost, s), "D2H records")) ||
-        (st = hip_check(hipMemcpyAsync(&nprod, d_nprod.as<int64_t>() + nq - 1, 8, hipMemcpyDeviceToHost, s), "D2H products")) ||
-        (st = hip_check(hipMemcpyAsync(&nload, d_nload.as<int64_t>() + nq - 1, 8, hipMemcpyDeviceToHost, s), "D2H loads")) ||
-        (st = hip_check(hipStreamSynchronize(s), "entry records")))
-      return st;
-    tp.n_prod = nprod;
-    tp.n_loads = nload;
-    if (nprod != n)
-      return set_errorf(CQMM_ERR_STATE, "tile plan: %lld listed products for %lld triplets", (long long)nprod,
-                        (long long)n);
-    // The kernel reads 64 words at a time.
-    if ((st = tp.prod.alloc(((size_t)nrec + 64) * 4))) return st;
-    if ((st = hip_check(hipMemsetAsync(tp.prod.as<uint32_t>() + nrec, 0, 64 * 4, s), "memset records tail"))) return st;
-    hipLaunchKernelGGL((k_wave_records<true>), grid, dim3(256), 0, s, d_src.as<int32_t>(), tp.n_wave,
-                       8, tp.wave_out.as<int32_t>(), d_tebeg.as<int32_t>(), d_ep.as<int32_t>(), d_eq.as<int32_t>(),
-                       nullptr, nullptr, nullptr, tp.pstart.as<int64_t>(), tp.prod.as<uint32_t>());
-    if ((st = hip_check(hipGetLastError(), "tile builder launch"))) return st;
-    st = hip_check(hipStreamSynchronize(s), "tile build");
-    pt.mark("  tiles: entry records");
+  // Entry records of the quadrants: count, first record of each, fill.
+  const size_t nq = src.size();
+  DevBuf d_src, d_nrec, d_nprod, d_nload;
+  if ((st = d_src.alloc(nq * 4)) || (st = d_nrec.alloc(nq * 8)) || (st = d_nprod.alloc(nq * 8)) ||
+      (st = d_nload.alloc(nq * 8)) || (st = tp.pstart.alloc((nq + 1) * 8)))
     return st;
-  }
-  if ((st = tp.list.alloc(nl * 4))) return st;
-  hipLaunchKernelGGL(k_list_fill, dim3(grid1(ne, 256)), dim3(256), 0, s, d_ep.as<int32_t>(), d_eq.as<int32_t>(),
-                     d_elbeg.as<int64_t>(), ne, tp.list.as<int32_t>());
-  // Chunks.
-  hipLaunchKernelGGL((k_chunks<false>), dim3(grid1(in.n_tiles, 256)), dim3(256), 0, s, d_tebeg.as<int32_t>(),
-                     d_emask.as<uint32_t>(), in.n_tiles, cap, kDenseEntries, nullptr, d_nch.as<int32_t>());
-  if ((st = tp.tile_chunk.alloc(((size_t)in.n_tiles + 1) * 4))) return st;
-  if ((st = hip_check(hipMemsetAsync(tp.tile_chunk.p, 0, 4, s), "memset tile_chunk"))) return st;
-  if ((st = inclusive_scan(d_nch.as<int32_t>(), tp.tile_chunk.as<int32_t>() + 1, (size_t)in.n_tiles, s))) return st;
-  int32_t nch = 0;
-  if ((st = hip_check(hipMemcpyAsync(&nch, tp.tile_chunk.as<int32_t>() + in.n_tiles, 4, hipMemcpyDeviceToHost, s),
-                      "D2H chunks")) ||
-      (st = hip_check(hipStreamSynchronize(s), "chunk count")))
+  if ((st = hip_check(hipMemcpyAsync(d_src.p, src.data(), nq * 4, hipMemcpyHostToDevice, s), "H2D quadrants"))) return st;
+  const dim3 grid(grid1((int64_t)nq, 4));
+  auto *count = tp.dense ? &k_wave_records<false, true> : &k_wave_records<false, false>;
+  hipLaunchKernelGGL(count, grid, dim3(256), 0, s, d_src.as<int32_t>(), tp.n_wave, tp.wave_out.as<int32_t>(), d_tebeg.as<int32_t>(), d_ep.as<int32_t>(), d_eq.as<int32_t>(),
+                     d_nrec.as<int64_t>(), d_nprod.as<int64_t>(), d_nload.as<int64_t>(), nullptr, nullptr);
+  int64_t nrec = 0, nprod = 0, nload = 0;
+  if ((st = hip_check(hipMemsetAsync(tp.pstart.p, 0, 8, s), "memset pstart")) ||
+      (st = inclusive_scan(d_nrec.as<int64_t>(), tp.pstart.as<int64_t>() + 1, nq, s)) ||
+      (st = inclusive_scan(d_nprod.as<int64_t>(), d_nprod.as<int64_t>(), nq, s)) ||
+      (st = inclusive_scan(d_nload.as<int64_t>(), d_nload.as<int64_t>(), nq, s)) ||
+      (st = hip_check(hipMemcpyAsync(&nrec, tp.pstart.as<int64_t>() + nq, 8, hipMemcpyDeviceToHost, s), "D2H records")) ||
+      (st = hip_check(hipMemcpyAsync(&nprod, d_nprod.as<int64_t>() + nq - 1, 8, hipMemcpyDeviceToHost, s), "D2H products")) ||
+      (st = hip_check(hipMemcpyAsync(&nload, d_nload.as<int64_t>() + nq - 1, 8, hipMemcpyDeviceToHost, s), "D2H loads")) ||
+      (st = hip_check(hipStreamSynchronize(s), "entry records")))
     return st;
-  tp.n_chunks = nch;
-  DevBuf d_centry;
-  if ((st = d_centry.alloc(((size_t)nch + 1) * 4))) return st;
-  hipLaunchKernelGGL((k_chunks<true>), dim3(grid1(in.n_tiles, 256)), dim3(256), 0, s, d_tebeg.as<int32_t>(),
-                     d_emask.as<uint32_t>(), in.n_tiles, cap, kDenseEntries, tp.tile_chunk.as<int32_t>(),
-                     d_centry.as<int32_t>());
-  if ((st = hip_check(hipMemcpyAsync(d_centry.as<int32_t>() + nch, &ne32, 4, hipMemcpyHostToDevice, s),
-                      "H2D chunk end")))
-    return st;
-  if ((st = tp.chunk_lbeg.alloc(((size_t)nch + 1) * 8))) return st;
-  hipLaunchKernelGGL(k_chunk_lbeg, dim3(grid1((int64_t)nch + 1, 256)), dim3(256), 0, s, d_centry.as<int32_t>(),
-                     d_elbeg.as<int64_t>(), (int64_t)nch + 1, tp.chunk_lbeg.as<int64_t>());
-  if ((st = d_ecoff.alloc((size_t)ne * 4))) return st;
-  hipLaunchKernelGGL(k_entry_coff, dim3(grid1((int64_t)nch, 256)), dim3(256), 0, s, d_centry.as<int32_t>(),
-                     d_elbeg.as<int64_t>(), (int64_t)nch, d_ecoff.as<int32_t>());
-  pt.mark("  tiles: entries + chunks");
-  // The dense kernel reads the entries themselves.
-  tp.chunk_entry = std::move(d_centry);
-  tp.entry_mask = std::move(d_emask);
-  tp.entry_coff = std::move(d_ecoff);
-  tp.n_prod = n;
+  tp.n_prod = nprod;
+  tp.n_loads = nload;
+  if (nprod != n)
+    return set_errorf(CQMM_ERR_STATE, "tile plan: %lld listed products for %lld triplets", (long long)nprod,
+                      (long long)n);
+  // The kernels read 64 words at a time, k_quad4 64 ahead (no block: -1).
+  if ((st = tp.prod.alloc(((size_t)nrec + kWavePad) * 4))) return st;
+  if ((st = hip_check(hipMemsetAsync(tp.prod.as<uint32_t>() + nrec, 0xff, kWavePad * 4, s), "memset records tail"))) return st;
+  auto *fill = tp.dense ? &k_wave_records<true, true> : &k_wave_records<true, false>;
+  hipLaunchKernelGGL(fill, grid, dim3(256), 0, s, d_src.as<int32_t>(), tp.n_wave, tp.wave_out.as<int32_t>(), d_tebeg.as<int32_t>(), d_ep.as<int32_t>(), d_eq.as<int32_t>(),
+                     nullptr, nullptr, nullptr, tp.pstart.as<int64_t>(), tp.prod.as<uint32_t>());
   if ((st = hip_check(hipGetLastError(), "tile builder launch"))) return st;
-  return hip_check(hipStreamSynchronize(s), "tile build");
+  st = hip_check(hipStreamSynchronize(s), "tile build");
+  pt.mark("  tiles: entry records");
+  return st;
 }
 
 int launch_tile_products(const TilePlan &tp, bool q_trans, const double *P, const double *Q, double *O,
