@@ -382,9 +382,9 @@ int cqmm_matrix_product(cqmm_ctx *ctx, int32_t A, int32_t B, int32_t C, int32_t 
     // FP64 launch above.
     if (hlen(ctx, A) < tp.len_p || hlen(ctx, B) < tp.len_q || hlen(ctx, C) < tp.len_out)
       return cq::set_errorf(CQMM_ERR_STATE, "cqmm_matrix_product: operand lengths below mult %d's", mult_id);
-    void *fp, *fq, *fo;
+    void *fp, *fq, *fo = nullptr;
     if ((st = get_scratch(ctx, "prodP", tp.len_p * 4, &fp)) || (st = get_scratch(ctx, "prodQ", tp.len_q * 4, &fq)) ||
-        (st = get_scratch(ctx, "prodO", tp.len_out * 4, &fo)))
+        (!cq::f32_writes_f64(tp) && (st = get_scratch(ctx, "prodO", tp.len_out * 4, &fo))))
       return st;
     // Split-BF16 x3 where the plan's kernel has it, else FP32 MFMA with FP64 sums.
     const int mode = (ctx->product_precision == 4 && !(cq::uses_tiles(tp) && cq::tiles_take_bf16x3(tp.tiles)))
@@ -396,9 +396,8 @@ int cqmm_matrix_product(cqmm_ctx *ctx, int32_t A, int32_t B, int32_t C, int32_t 
       if ((st = cq::op_to_f32(tp.len_p, dptr(ctx, A), (float *)fp, s))) return st;
       if ((st = cq::op_to_f32(tp.len_q, dptr(ctx, B), (float *)fq, s))) return st;
     }
-    if ((st = cq::launch_block_products_f32(tp, (const float *)fp, (const float *)fq, (float *)fo, mode, s)))
-      return st;
-    return cq::op_to_f64(tp.len_out, (const float *)fo, dptr(ctx, C), s);
+    return cq::launch_block_products_f32_to_f64(tp, (const float *)fp, (const float *)fq, (float *)fo, dptr(ctx, C),
+                                                mode, s);
   });
 }
 

@@ -124,6 +124,7 @@ struct TileArgs {
   const void *P, *Q;
   void *O;
   int32_t n_tiles, tile_base;
+  int32_t wide;                 // FP32 modes: O is FP64 (the FP32 results, widened)
 };
 // Up to kMaxGroup products in one grouped launch, passed by value (kernel
 // argument memory, 2.7 KB).
@@ -231,6 +232,14 @@ int launch_block_products(const TripletPlan &tp, const double *P, const double *
 // `mode` (1, 2 or 3, as for launch_tile_products_f32).
 int launch_block_products_f32(const TripletPlan &tp, const float *P, const float *Q, float *O, int mode,
                               hipStream_t stream);
+// The same with the FP32 result widened to FP64 in O. Kernels of the uniform
+// sizes write O themselves (f32_writes_f64; O32 is not used and may be null),
+// the others write O32 [len_out], which is then widened: 13x13 split BF16, 1024
+// atoms, 5.0 ms with the widening pass, 4.2 ms without.
+bool tiles_write_f64(const TilePlan &tp);
+bool f32_writes_f64(const TripletPlan &tp);
+int launch_block_products_f32_to_f64(const TripletPlan &tp, const float *P, const float *Q, float *O32, double *O,
+                                     int mode, hipStream_t stream);
 // Symmetric-result plans: write each mirrored block as the transpose of its
 // computed partner (FP64 or FP32 result); nothing for other plans.
 // launch_block_products(_f32) call it; callers that launch a plan's tile

@@ -308,6 +308,7 @@ int McwEngine::products(int which) {
     const void *P, *Q;
     void *O;
     int mode = 0;
+    bool wide = false;
     if (j.fp32_phase) {
       float *A32 = which == 0 ? j.L32 : which == 1 ? j.LS32 : j.LSL32;
       float *B32 = which == 0 ? j.S32 : which == 1 ? j.L32 : j.LS32;
@@ -316,6 +317,9 @@ int McwEngine::products(int which) {
       Q = B32;
       O = C32;
       mode = j.mode;
+      // LSLSL is only read in FP64.
+      wide = which == 2 && f32_writes_f64(tp);
+      if (wide) O = dptr(ctx, C);
     } else {
       P = dptr(ctx, A);
       Q = dptr(ctx, B);
@@ -326,17 +330,19 @@ int McwEngine::products(int which) {
       else MTRY(launch_block_products_f32(tp, (const float *)P, (const float *)Q, (float *)O, mode, s_));
       continue;
     }
-    if (tp.n_mirror > 0) mirrors.push_back({&tp, O, mode != 0});
+    if (tp.n_mirror > 0) mirrors.push_back({&tp, O, mode != 0 && !wide});
     if (tp.tiles.n_tiles == 0) continue;
+    TileArgs ta = tile_launch_args(tp.tiles, P, Q, O);
+    ta.wide = wide;
     if (!group_) {
-      MTRY(launch_tile_args(tp.tiles, tp.q_trans, mode, tile_launch_args(tp.tiles, P, Q, O), s_));
+      MTRY(launch_tile_args(tp.tiles, tp.q_trans, mode, ta, s_));
       continue;
     }
     Grp &g = groups[tile_group_key(tp.tiles, tp.q_trans, mode)];
     g.tp = &tp.tiles;
     g.qt = tp.q_trans;
     g.mode = mode;
-    g.a.push_back(tile_launch_args(tp.tiles, P, Q, O));
+    g.a.push_back(ta);
   }
   for (auto &kv : groups) {
     Grp &g = kv.second;
@@ -393,7 +399,8 @@ int McwEngine::enqueue_step() {
     double *sc = dsc(j);
     if (j.fp32_phase) {
       if (j.mode != 4) MTRY(op_to_f64(hlen(ctx, j.LSL), j.LSL32, dptr(ctx, j.LSL), s_));
-      MTRY(op_to_f64(hlen(ctx, j.LSLSL), j.LSLSL32, dptr(ctx, j.LSLSL), s_));
+      if (!f32_writes_f64(ctx->mults.at(j.su.mult_LSL_SL_L).plan->tp))
+        MTRY(op_to_f64(hlen(ctx, j.LSLSL), j.LSLSL32, dptr(ctx, j.LSLSL), s_));
     }
     // c1 = Tr[S (LSL - LSLSL)] and c2 = Tr[S (L - LSL)] on the S range.
     MTRY(op_scale(hlen(ctx, j.top), 0.0, dptr(ctx, j.top), s_));

@@ -25,6 +25,7 @@
 #include "../../include/cqmm.h"
 #include "cq_common.h"
 #include "cq_device.h"
+#include "cq_ops.h"
 
 namespace {
 
@@ -366,6 +367,22 @@ int launch_block_products_f32(const TripletPlan &tp, const float *P, const float
                               hipStream_t s) {
   const int st = products_f32(tp, P, Q, O, mode, s);
   return st ? st : mirror_result_f32(tp, O, s);
+}
+
+bool f32_writes_f64(const TripletPlan &tp) { return uses_tiles(tp) && tiles_write_f64(tp.tiles); }
+
+int launch_block_products_f32_to_f64(const TripletPlan &tp, const float *P, const float *Q, float *O32, double *O,
+                                     int mode, hipStream_t s) {
+  int st;
+  if (!f32_writes_f64(tp)) {
+    if ((st = launch_block_products_f32(tp, P, Q, O32, mode, s))) return st;
+    return op_to_f64(tp.len_out, O32, O, s);
+  }
+  if (mode < 1 || mode > 4) return set_errorf(CQMM_ERR_ARG, "block products: FP32 mode %d", mode);
+  TileArgs a = tile_launch_args(tp.tiles, P, Q, O);
+  a.wide = 1;
+  if ((st = launch_tile_args(tp.tiles, tp.q_trans, mode, a, s))) return st;
+  return mirror_result(tp, O, s);
 }
 
 int launch_block_products(const TripletPlan &tp, const double *P, const double *Q, double *O, bool fp32,

@@ -89,8 +89,7 @@ int cqmm_mat_mult_fp32_noalloc(cqmm_plan *plan, double *a, int64_t lena, const d
       if ((st = cq::op_to_f32(tp.len_p, dP, fp, s))) return st;
       if ((st = cq::op_to_f32(tp.len_q, b, fq, s))) return st;
     }
-    if ((st = cq::launch_block_products_f32(tp, fp, fq, fo, mode, s))) return st;
-    if ((st = cq::op_to_f64(tp.len_out, fo, dO, s))) return st;
+    if ((st = cq::launch_block_products_f32_to_f64(tp, fp, fq, fo, dO, mode, s))) return st;
     if (!(flags & CQMM_NO_SYNC)) return cq::hip_check(hipStreamSynchronize(s), "cqmm_mat_mult_fp32_noalloc");
     return CQMM_OK;
   });

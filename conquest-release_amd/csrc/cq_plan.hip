@@ -1308,11 +1308,12 @@ int cqmm_mat_mult(cqmm_plan *plan, double *a, int64_t lena, const double *b, int
     if (!fp32) {
       st = cq::launch_block_products(plan->tp, dP, db, dO, false, s);
     } else {
-      // FP32 products on FP32 copies; the result is widened back into the FP64 array.
+      // FP32 products on FP32 copies; the result widened into the FP64 array.
       const cq::TripletPlan &tp = plan->tp;
       if (plan->fp.bytes < (size_t)tp.len_p * 4 && (st = plan->fp.alloc(tp.len_p * 4))) return st;
       if (plan->fq.bytes < (size_t)tp.len_q * 4 && (st = plan->fq.alloc(tp.len_q * 4))) return st;
-      if (plan->fo.bytes < (size_t)tp.len_out * 4 && (st = plan->fo.alloc(tp.len_out * 4))) return st;
+      if (!cq::f32_writes_f64(tp) && plan->fo.bytes < (size_t)tp.len_out * 4 && (st = plan->fo.alloc(tp.len_out * 4)))
+        return st;
       const int mode = (flags & CQMM_BF16X3) ? 4 : (flags & CQMM_FP32_RUN64) ? 3 : (flags & CQMM_FP32_ACC64) ? 2 : 1;
       if (mode == 4) {
         if ((st = cq::op_to_bf16x2(tp.len_p, dP, plan->fp.as<uint32_t>(), s))) return st;
@@ -1321,10 +1322,8 @@ int cqmm_mat_mult(cqmm_plan *plan, double *a, int64_t lena, const double *b, int
         if ((st = cq::op_to_f32(tp.len_p, dP, plan->fp.as<float>(), s))) return st;
         if ((st = cq::op_to_f32(tp.len_q, db, plan->fq.as<float>(), s))) return st;
       }
-      if ((st = cq::launch_block_products_f32(tp, plan->fp.as<float>(), plan->fq.as<float>(), plan->fo.as<float>(),
-                                              mode, s)))
-        return st;
-      st = cq::op_to_f64(tp.len_out, plan->fo.as<float>(), dO, s);
+      st = cq::launch_block_products_f32_to_f64(tp, plan->fp.as<float>(), plan->fq.as<float>(), plan->fo.as<float>(),
+                                                dO, mode, s);
     }
     if (st) return st;
     if (!dev) {

@@ -276,7 +276,8 @@ __device__ inline void wait_blocks(int32_t after) {
 // per chunk; the busiest wavefront has 1.25 to 1.56 times the mean products):
 // 13x13 FP64 4096 atoms type 2 50.2 -> 46.0 ms, 1024 atoms symmetric
 // 15.9 -> 15.3 ms, 9x9 FP32 with FP64 sums 1500 atoms 11.1 -> 8.9 ms, 13x13 split
-// BF16 1024 atoms 5.9 -> 5.0 ms, 9x9 FP64 60 atoms (one LNV solve) 12.5 -> 10.0 ms.
+// BF16 1024 atoms 5.9 -> 5.0 ms (4.2 ms with the FP64 result written here, not
+// widened by a pass of its own), 9x9 FP64 60 atoms (one LNV solve) 12.5 -> 10.0 ms.
 // Tried and slower: operands straight to registers (4096 atoms 58 ms: 18 to 33
 // address cycles per load), two stages instead of the ring (split BF16 6.2 ms),
 // three wavefronts per SIMD with right operands read per product (9x9 11.1 ms).
@@ -300,7 +301,6 @@ k_wave_products(const ARG arg) {
   if (tile < 0) return;
   const int lane = threadIdx.x, r = lane & 15, g = lane >> 4;
   const char *P = static_cast<const char *>(a.P), *Q = static_cast<const char *>(a.Q);
-  T *__restrict__ O = static_cast<T *>(a.O);
   // The tile's output blocks (-1: none): bit 4*row + column of `valid`.
   const int32_t *wo = a.wave_out + (int64_t)tile * 16;
   const uint32_t valid = (uint32_t)__ballot(wo[r] >= 0) & 0xffffu;
@@ -453,16 +453,20 @@ k_wave_products(const ARG arg) {
       while (fits()) issue();
     } while (nq > 0);
   }
+  auto write = [&](auto *out) {
 #pragma unroll
-  for (int u = 0; u < 16; ++u) {
-    if (!(valid >> u & 1u)) continue;
-    T *o = O + (int64_t)wo[u] * NS2 + NSF * r;
+    for (int u = 0; u < 16; ++u) {
+      if (!(valid >> u & 1u)) continue;
+      auto *o = out + (int64_t)wo[u] * NS2 + NSF * r;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = MODE == 0 ? g + 4 * i : 4 * g + i;
-      if (r < NSF && row < NSF) o[row] = MODE == 1 ? (T)a32[u][i] : (T)a64[u][i];
+      for (int i = 0; i < 4; ++i) {
+        const int row = MODE == 0 ? g + 4 * i : 4 * g + i;
+        if (r < NSF && row < NSF) o[row] = MODE == 1 ? (T)a32[u][i] : (T)a64[u][i];
+      }
     }
-  }
+  };
+  if (MODE != 0 && a.wide) write(static_cast<double *>(a.O));
+  else write(static_cast<T *>(a.O));
 }
 
 // 4x4 blocks: one wavefront computes 4x4 output blocks (a quadrant of a tile), on
@@ -498,7 +502,6 @@ __global__ void __launch_bounds__(64) k_quad4(const ARG arg) {
   const int32_t tile = tile_select(arg, a);
   if (tile < 0) return;
   const int lane = threadIdx.x, r = lane & 15, g = lane >> 4;
-  T *__restrict__ O = static_cast<T *>(a.O);
   dbl4 a64 = {0.0, 0.0, 0.0, 0.0};
   flt4 a32 = {0.f, 0.f, 0.f, 0.f};
   const int64_t w0 = a.pstart[tile];
@@ -558,12 +561,16 @@ __global__ void __launch_bounds__(64) k_quad4(const ARG arg) {
   // FP64 accumulator D[g+4e][r], FP32 D[4g+e][r]: quadrant row R, column r is
   // element (R % 4, r % 4) of block (R / 4, r / 4).
   const int32_t *wo = a.wave_out + (int64_t)tile * 16;
+  auto write = [&](auto *out) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int rq = MODE == 0 ? e : g, ri = MODE == 0 ? g : e;
-    const int32_t o = wo[rq * 4 + (r >> 2)];
-    if (o >= 0) O[(int64_t)o * 16 + ri + 4 * (r & 3)] = MODE == 1 ? (T)a32[e] : (T)a64[e];
-  }
+    for (int e = 0; e < 4; ++e) {
+      const int rq = MODE == 0 ? e : g, ri = MODE == 0 ? g : e;
+      const int32_t o = wo[rq * 4 + (r >> 2)];
+      if (o >= 0) out[(int64_t)o * 16 + ri + 4 * (r & 3)] = MODE == 1 ? (T)a32[e] : (T)a64[e];
+    }
+  };
+  if (MODE != 0 && a.wide) write(static_cast<double *>(a.O));
+  else write(static_cast<T *>(a.O));
 }
 
 // ---------------------------------------------------------------- builder
@@ -1676,6 +1683,8 @@ int launch_tile_products_f32(const TilePlan &tp, bool q_trans, const float *P, c
   if (tp.n_tiles == 0) return CQMM_OK;
   return launch_tile_args(tp, q_trans, mode, tile_launch_args(tp, P, Q, O), s);
 }
+
+bool tiles_write_f64(const TilePlan &tp) { return tp.n_wave > 0; }
 
 TileArgs tile_launch_args(const TilePlan &tp, const void *P, const void *Q, void *O) {
   TileArgs a;
