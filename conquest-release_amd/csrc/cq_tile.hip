@@ -116,13 +116,21 @@ using cq::TileArgs;
 using cq::TileGroup;
 using cq::kMaxGroup;
 
-// Tile of this workgroup, XCD-aware: workgroup b runs on XCD b % 8 and takes
-// tile (b % 8) * ceil(T/8) + b / 8, so neighbouring tiles (same rows) share an
-// L2. Returns -1 past the last tile.
+// Tile of this workgroup, XCD-aware: workgroup b runs on XCD b % 8, and
+// kXcdRun consecutive tiles (same rows) go to one XCD, whose L2 they share,
+// before the next kXcdRun go to the next XCD; the tiles after the last full
+// round are split evenly. One run of a eighth of all tiles per XCD keeps the
+// XCDs apart in memory and leaves them with unequal work: 13x13 symmetric 1024
+// atoms 15.2 ms, with runs of 128 13.7, 512 13.4, 2048 13.5, 8192 13.4 ms.
+// Returns -1 past the last tile.
+constexpr int32_t kXcdRun = 512;
 __device__ inline int32_t xcd_tile(int32_t n) {
-  const int32_t per = (n + 7) >> 3;
-  const int32_t t = (int32_t)(blockIdx.x & 7) * per + (int32_t)(blockIdx.x >> 3);
-  return t < n ? t : -1;
+  const int32_t x = (int32_t)(blockIdx.x & 7), i = (int32_t)(blockIdx.x >> 3);
+  const int32_t full = n / (8 * kXcdRun);
+  if (i < full * kXcdRun) return i / kXcdRun * (8 * kXcdRun) + x * kXcdRun + i % kXcdRun;
+  const int32_t done = full * (8 * kXcdRun), per = (n - done + 7) >> 3, k = i - full * kXcdRun;
+  const int32_t t = done + x * per + k;
+  return k < per && t < n ? t : -1;
 }
 
 __device__ inline int32_t tile_select(const TileArgs &arg, TileArgs &a) {
