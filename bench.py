@@ -65,14 +65,14 @@ def species_nsf(natoms, mix, seed):
     return vals[rng.choice(len(vals), size=natoms, p=probs / probs.sum())]
 
 
-TILE_KERNELS = {1: "k_tile_dense4_f64", 2: "k_tile_dense_mx_f64", 3: "k_tile_mixed_f64", 5: "k_tile_quad_f64"}
+TILE_KERNELS = {1: "k_quad4_f64", 2: "k_tile_dense_mx_f64", 3: "k_tile_mixed_f64", 5: "k_tile_quad_f64"}
 
 
 def kernel_name(info, nsf):
     """Name of the FP64 product kernel a plan runs (as rocprofv3 lists it, shortened)."""
     mixed = not isinstance(nsf, int)
     if info.kernel == cqmm.KERNEL_TILE:
-        return TILE_KERNELS.get(info.tile_family, "k_tile_products_f64")
+        return TILE_KERNELS.get(info.tile_family, "k_wave_products_f64")
     return "k_block_products_f64" if mixed else "k_block_products_f64_u"
 
 

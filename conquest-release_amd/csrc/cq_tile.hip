@@ -1176,7 +1176,7 @@ __global__ void __launch_bounds__(kTileThreads) k_tile_mixed(
 }
 
 // Mixed block sizes of at most 4x4 (e.g. C and H with single-zeta bases):
-// the dense-quadrant scheme of k_tile_dense4 over the mixed-size schedule.
+// the dense-quadrant scheme of one matrix step per entry over the mixed-size schedule.
 // Wavefront w owns quadrant (w / 2, w % 2) of the tile (4x4 blocks, each
 // inside a 4x4 corner of the quadrant's 16x16 MFMA tile) and issues one
 // 16x16x4 MFMA per entry: lane (r, g) supplies element (r % 4, g) of
