@@ -119,11 +119,12 @@ using cq::kMaxGroup;
 // Tile of this workgroup, XCD-aware: workgroup b runs on XCD b % 8, and
 // kXcdRun consecutive tiles (same rows) go to one XCD, whose L2 they share,
 // before the next kXcdRun go to the next XCD; the tiles after the last full
-// round are split evenly. One run of a eighth of all tiles per XCD keeps the
-// XCDs apart in memory and leaves them with unequal work: 13x13 symmetric 1024
-// atoms 15.2 ms, with runs of 128 13.7, 512 13.4, 2048 13.5, 8192 13.4 ms.
+// round are split evenly. With an eighth of all tiles per XCD their work is
+// unequal: 13x13 symmetric 1024 atoms 15.3 ms, with runs of 128 13.7, of 512 to
+// 8192 13.5 ms; short runs cost the smaller products (13x13 McWeeny of 128 atoms:
+// runs of 64 116 ms, 512 113, 8192 110).
 // Returns -1 past the last tile.
-constexpr int32_t kXcdRun = 512;
+constexpr int32_t kXcdRun = 8192;
 __device__ inline int32_t xcd_tile(int32_t n) {
   const int32_t x = (int32_t)(blockIdx.x & 7), i = (int32_t)(blockIdx.x >> 3);
   const int32_t full = n / (8 * kXcdRun);
