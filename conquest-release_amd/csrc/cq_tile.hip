@@ -541,6 +541,9 @@ __global__ void __launch_bounds__(64) k_quad4(const ARG arg) {
 #pragma unroll
     for (int i = 0; i < AHEAD; ++i) copy(w, i, i);
     for (int32_t rec = 0; rec < n; rec += 8) {
+      // The load of wn stays between the copies before it and those after it:
+      // the waits below count on that order.
+      asm volatile("" ::: "memory");
       const uint32_t wn = words[8 * (int64_t)(rec + 8)];
       asm volatile("" ::: "memory");
 #pragma unroll
@@ -548,7 +551,8 @@ __global__ void __launch_bounds__(64) k_quad4(const ARG arg) {
         if (rec + i >= n) break;
         copy(i + AHEAD < 8 ? w : wn, (i + AHEAD) & 7, (i + AHEAD) & 3);
         asm volatile("" ::: "memory");
-        // The record's copy is older than AHEAD others and, at first, the load of wn.
+        // The record's copy is older than AHEAD others and, for the first AHEAD
+        // records of the eight, the load of wn.
         if (i < AHEAD) __builtin_amdgcn_s_waitcnt((AHEAD + 1) | 0xf70);
         else __builtin_amdgcn_s_waitcnt(AHEAD | 0xf70);
         asm volatile("" ::: "memory");
