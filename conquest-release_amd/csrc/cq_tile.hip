@@ -174,8 +174,10 @@ struct Frag {
   static constexpr bool R1 = MODE != 4 && NSF % 4 == 1;  // the last contraction index on the VALU
   static constexpr int KM = MODE == 4 ? 4 : (R1 ? KS - 1 : KS);  // registers of the matrix steps
   static_assert(NSF % 4 <= 1, "block sizes 4m and 4m + 1");
-  T k[KM];    // element of each matrix step (MODE 4: hi and lo operands, two registers each)
-  T last[4];  // R1: left, A[row][NSF-1] of the lane's 4 accumulator rows; right, B[NSF-1][r] in last[0]
+  // A lane's accumulator rows that can lie in a block (FP64 g + 4e, FP32 4g + e).
+  static constexpr int ROWS = MODE == 0 ? KS : 4;
+  T k[KM];       // element of each matrix step (MODE 4: hi and lo operands, two registers each)
+  T last[ROWS];  // R1: left, A[row][NSF-1] of these rows; right, B[NSF-1][r] in last[0]
 };
 
 // A block's bytes go to LDS 16 per lane; where they end inside the last lane's
@@ -216,24 +218,35 @@ struct FragOff {
     for (int i = 0; i < F::KM; ++i) f.k[i] = blk[first[N == 1 ? 0 : i] + (N == 1 ? STEP * i : 0)];
     if constexpr (F::R1) {
 #pragma unroll
-      for (int e = 0; e < (RIGHT ? 1 : 4); ++e)
+      for (int e = 0; e < (RIGHT ? 1 : F::ROWS); ++e)
         f.last[e] = blk[last + (MODE == 0 ? 4 * e + (!RIGHT && 4 * e == NSF - 1 ? SHIFT : 0) : e)];
     }
     if constexpr (MODE == 4) split_words<NSF>(f.k, g);
   }
 };
 
+// Wavefronts per SIMD. FP64 blocks of 13 and 16: two, with all operands of a record
+// in registers. The others: three, with the left operands of one row at a time.
+// FP64 9x9 needs the third to cover a record's scalar work, as its matrix steps
+// are short: 2000 atoms, C(16 A) = A(8 A).B(12 A), 10.3 ms with two, 7.9 with three.
+constexpr int wave_per_simd(int mode, int nsf) { return mode == 0 && nsf > 9 ? 2 : 3; }
 // Ring of operand blocks of a wavefront: what its share of the 160 KB LDS
-// holds beside the record words, with 2 wavefronts per SIMD (FP64) or 3.
+// holds beside the record words.
 constexpr int kWaveWords = 256;  // record words in LDS
 constexpr int kWavePad = 128;    // words after a plan's last record
-constexpr int wave_per_simd(int mode) { return mode == 0 ? 2 : 3; }
 constexpr int wave_dmas(int nsf, int size) { return (nsf * nsf * size + 1023) / 1024; }  // copies per block
 constexpr int wave_ring(int mode, int nsf) {
   const int size = mode == 0 ? 8 : 4;
-  const int r = ((mode == 0 ? 20480 : 12800) - 4 * kWaveWords) / wave_stride(nsf, size);
+  const int r = ((wave_per_simd(mode, nsf) == 2 ? 20480 : 12800) - 4 * kWaveWords) / wave_stride(nsf, size);
   const int v = 63 / wave_dmas(nsf, size);  // the wait counts at most 63 copies
   return (r < v ? r : v) < 28 ? (r < v ? r : v) : 28;
+}
+
+// The lane, worked out where it is needed and not held in a register until then.
+__device__ inline int lane_again() {
+  uint32_t ones = ~0u;
+  asm volatile("" : "+s"(ones));
+  return (int)__builtin_amdgcn_mbcnt_hi(ones, __builtin_amdgcn_mbcnt_lo(ones, 0u));
 }
 
 // One operand block from memory to LDS. `lane16`: 16 * lane, and `end16` that of
@@ -295,7 +308,7 @@ __device__ inline void wait_blocks(int32_t after) {
 // fused multiply-adds after the matrix steps; a matrix step with three zeroed
 // indices takes 72 cycles in FP64).
 template <int MODE, bool QT, int NSF, class ARG>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(wave_per_simd(MODE))))
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(wave_per_simd(MODE, NSF))))
 k_wave_products(const ARG arg) {
   using F = Frag<MODE, NSF>;
   using T = typename F::T;
@@ -304,6 +317,8 @@ k_wave_products(const ARG arg) {
   constexpr int LB = wave_stride(NSF, (int)sizeof(T));
   constexpr int RING = wave_ring(MODE, NSF), PER = wave_dmas(NSF, (int)sizeof(T));
   static_assert(RING >= 8, "the ring holds every record");
+  constexpr bool ALL_LEFT = wave_per_simd(MODE, NSF) == 2;  // left operands of the record in registers, or of a row
+  constexpr bool TIGHT = MODE == 0 && !ALL_LEFT;            // every register of the three wavefronts' share is used
   __shared__ __attribute__((aligned(16))) char lds[RING * LB + 4 * kWaveWords];
   TileArgs a;
   const int32_t tile = tile_select(arg, a);
@@ -344,6 +359,7 @@ k_wave_products(const ARG arg) {
     char *wring = lds + RING * LB;
     auto piece = [&](int32_t j) {
       if (64 * j >= nw) return;
+      if constexpr (TIGHT) l4 = 4u * (uint32_t)lane_again();
       asm volatile("" : "+v"(l4));
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(words + 256 * (int64_t)j + l4),
                                        (__attribute__((address_space(3))) void *)(wring + 256 * (j & 3)), 4, 0, 0);
@@ -352,7 +368,7 @@ k_wave_products(const ARG arg) {
     uint32_t win;
     auto refill = [&]() {
       base = at;
-      win = ((const uint32_t *)wring)[(at + lane) % kWaveWords];
+      win = ((const uint32_t *)wring)[(at + (TIGHT ? lane_again() : lane)) % kWaveWords];
     };
     auto word = [&](int32_t i) { return (uint32_t)__builtin_amdgcn_readlane((int)win, i - base); };
     for (int32_t j = 0; j < 4; ++j) piece(j);
@@ -410,8 +426,8 @@ k_wave_products(const ARG arg) {
         oQ.load((const T *)(lds + pq), g, right[k]);
         step(pq, 1);
       }
-      F left[MODE == 0 ? 4 : 1];
-      if constexpr (MODE == 0) {
+      F left[ALL_LEFT ? 4 : 1];
+      if constexpr (ALL_LEFT) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           if (!(m >> u & 1u)) continue;
@@ -422,11 +438,11 @@ k_wave_products(const ARG arg) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         if (!(m >> u & 1u)) continue;
-        if constexpr (MODE != 0) {
+        if constexpr (!ALL_LEFT) {
           oP.load((const T *)(lds + head), g, left[0]);
           step(head, 1);
         }
-        const F &x = left[MODE == 0 ? u : 0];
+        const F &x = left[ALL_LEFT ? u : 0];
         const uint32_t todo = (valid >> (4 * u)) & cols;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -438,7 +454,7 @@ k_wave_products(const ARG arg) {
             for (int i = 0; i < F::KM; ++i) d = __builtin_amdgcn_mfma_f64_16x16x4f64(x.k[i], y.k[i], d, 0, 0, 0);
             if constexpr (F::R1) {
 #pragma unroll
-              for (int i = 0; i < 4; ++i) d[i] = __builtin_fma(x.last[i], y.last[0], d[i]);
+              for (int i = 0; i < F::ROWS; ++i) d[i] = __builtin_fma(x.last[i], y.last[0], d[i]);
             }
           } else {
             flt4 t = MODE == 1 ? a32[4 * u + k] : flt4{0.f, 0.f, 0.f, 0.f};
@@ -451,7 +467,7 @@ k_wave_products(const ARG arg) {
               for (int i = 0; i < F::KM; ++i) t = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[i], y.k[i], t, 0, 0, 0);
               if constexpr (F::R1) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) t[i] = __builtin_fmaf(x.last[i], y.last[0], t[i]);
+                for (int i = 0; i < F::ROWS; ++i) t[i] = __builtin_fmaf(x.last[i], y.last[0], t[i]);
               }
             }
             if constexpr (MODE == 1) {
@@ -468,15 +484,16 @@ k_wave_products(const ARG arg) {
       while (fits()) issue();
     } while (nq > 0);
   }
+  const int rw = TIGHT ? lane_again() & 15 : r, gw = TIGHT ? lane_again() >> 4 : g;
   auto write = [&](auto *out) {
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
       if (!(valid >> u & 1u)) continue;
-      auto *o = out + (int64_t)out_blk[u] * NS2 + NSF * r;
+      auto *o = out + (int64_t)out_blk[u] * NS2 + NSF * rw;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int row = MODE == 0 ? g + 4 * i : 4 * g + i;
-        if (r < NSF && row < NSF) o[row] = MODE == 1 ? (T)a32[u][i] : (T)a64[u][i];
+      for (int i = 0; i < F::ROWS; ++i) {
+        const int row = MODE == 0 ? gw + 4 * i : 4 * gw + i;
+        if (rw < NSF && row < NSF) o[row] = MODE == 1 ? (T)a32[u][i] : (T)a64[u][i];
       }
     }
   };

@@ -63,3 +63,23 @@ def test_results_are_written_without_waiting_for_loads(tile_code):
         assert not re.search(r"\b(global|flat|scratch)_load", code[stores:]), name
         seen += 1
     assert seen == len(names)
+
+
+def test_registers_and_lds_fit_the_wavefronts(tile_code):
+    """Two wavefronts per SIMD for FP64 blocks of 13 and 16, three for the others; no
+    scratch memory but, in split BF16, for a few lane constants around the loop."""
+    notes = subprocess.run([os.path.join(LLVM, "llvm-readelf"), "--notes", tile_code], capture_output=True, text=True,
+                           check=True).stdout
+    names = set(_wave_kernels(tile_code))
+    seen = 0
+    for kernel in notes.split("  - .agpr_count")[1:]:
+        field = dict(re.findall(r"^\s*\.(\w+):\s+(\S+)$", kernel, flags=re.M))
+        if field["name"] not in names:
+            continue
+        mode, nsf = map(int, re.search(r"k_wave_productsILi(\d+)ELb[01]ELi(\d+)E", field["name"]).groups())
+        waves = 2 if mode == 0 and nsf > 9 else 3
+        assert int(field["vgpr_count"]) <= 512 // waves // 8 * 8, (field["name"], field["vgpr_count"])
+        assert int(field["group_segment_fixed_size"]) * 4 * waves <= 160 * 1024, field["name"]
+        assert int(field["private_segment_fixed_size"]) <= (32 if mode == 4 else 0), field["name"]
+        seen += 1
+    assert seen == len(names)
