@@ -6,6 +6,8 @@
 #include <cstdint>
 #include <vector>
 
+#include "cq_split.h"
+
 namespace cq {
 
 struct Runtime {
@@ -89,6 +91,7 @@ struct TilePlan {
   bool dense = false;
   bool quad = false;   // class tiles (k_tile_quad): one row and one column block size per tile
   int32_t wgs = 0;     // class tiles: workgroups of a persistent launch (0: one per tile)
+  WorkParts parts;     // of the launch units, for their split over the XCDs
   DevBuf chunk_entry;  // int32 [n_chunks+1] first entry of each chunk
   DevBuf entry_mask;   // uint32 [n_entries] left-operand rows | right-operand columns << 8 present
   DevBuf entry_coff;   // int32 [n_entries] first operand block (mixed: element) of the entry in its chunk's stage
@@ -125,13 +128,20 @@ struct TileArgs {
   void *O;
   int32_t n_tiles, tile_base;
   int32_t wide;                 // FP32 modes: O is FP64 (the FP32 results, widened)
+  const TilePlan *plan;         // read by the launching host code only
+};
+// A launch of one product; XCD x runs the units [xcd[x], xcd[x + 1]).
+struct TileOne {
+  TileArgs a;
+  int32_t xcd[kXcds + 1];
 };
 // Up to kMaxGroup products in one grouped launch, passed by value (kernel
-// argument memory, 2.7 KB).
+// argument memory, 2.8 KB).
 constexpr int kMaxGroup = 16;
 struct TileGroup {
   TileArgs a[kMaxGroup];
-  int32_t ngrp, total;
+  int32_t ngrp, total;             // products; launch units of all
+  int32_t xcd[kXcds + 1];
 };
 
 // Triplet list of one product, grouped by output block (segment), each group in
@@ -213,7 +223,7 @@ int launch_tile_products_f32(const TilePlan &tp, bool q_trans, const float *P, c
 // launch (same summation order). mode: 0 FP64, else an FP32 mode (1, 2, 3).
 TileArgs tile_launch_args(const TilePlan &tp, const void *P, const void *Q, void *O);
 int tile_group_key(const TilePlan &tp, bool q_trans, int mode);
-int launch_tile_group(const TilePlan &tp, bool q_trans, int mode, const TileGroup &g, hipStream_t s);
+int launch_tile_group(const TilePlan &tp, bool q_trans, int mode, TileGroup &g, hipStream_t s);
 // One product's tile launch from its TileArgs (the launch cqmm_mat_mult makes).
 int launch_tile_args(const TilePlan &tp, bool q_trans, int mode, const TileArgs &a, hipStream_t s);
 

@@ -114,36 +114,42 @@ __device__ inline void dma_piece(const uint32_t *src, uint32_t *dst) {
 
 using cq::TileArgs;
 using cq::TileGroup;
+using cq::TileOne;
 using cq::kMaxGroup;
 
-// Tile of this workgroup, XCD-aware: workgroup b runs on XCD b % 8, and
-// kXcdRun consecutive tiles (same rows) go to one XCD, whose L2 they share,
-// before the next kXcdRun go to the next XCD; the tiles after the last full
-// round are split evenly. With an eighth of all tiles per XCD their work is
-// unequal: 13x13 symmetric 1024 atoms 15.3 ms, with runs of 128 13.7, of 512 to
-// 8192 13.5 ms; short runs cost the smaller products (13x13 McWeeny of 128 atoms:
-// runs of 64 116 ms, 512 113, 8192 110).
-// Returns -1 past the last tile.
-constexpr int32_t kXcdRun = 8192;
-__device__ inline int32_t xcd_tile(int32_t n) {
-  const int32_t x = (int32_t)(blockIdx.x & 7), i = (int32_t)(blockIdx.x >> 3);
-  const int32_t full = n / (8 * kXcdRun);
-  if (i < full * kXcdRun) return i / kXcdRun * (8 * kXcdRun) + x * kXcdRun + i % kXcdRun;
-  const int32_t done = full * (8 * kXcdRun), per = (n - done + 7) >> 3, k = i - full * kXcdRun;
-  const int32_t t = done + x * per + k;
-  return k < per && t < n ? t : -1;
+// Launch units [lo, hi) of this workgroup's XCD: workgroup b runs on XCD b % 8, and
+// each XCD takes consecutive units (same rows), which share its L2. All nine
+// bounds are read at fixed places of the arguments: one load indexed by the XCD
+// costs the mixed sizes 1.5% (4096 atoms 4/9/13 27.6 -> 28.0 ms).
+__device__ inline void xcd_units(const int32_t (&xcd)[cq::kXcds + 1], int32_t &lo, int32_t &hi) {
+  const int32_t x = (int32_t)(blockIdx.x & 7);
+  lo = xcd[0];
+  hi = xcd[1];
+#pragma unroll
+  for (int k = 1; k < cq::kXcds; ++k) {
+    lo = x == k ? xcd[k] : lo;
+    hi = x == k ? xcd[k + 1] : hi;
+  }
 }
 
-__device__ inline int32_t tile_select(const TileArgs &arg, TileArgs &a) {
-  a = arg;
-  return xcd_tile(a.n_tiles);
+// This workgroup's launch unit, -1 past its XCD's last.
+__device__ inline int32_t xcd_tile(const int32_t (&xcd)[cq::kXcds + 1]) {
+  int32_t lo, hi;
+  xcd_units(xcd, lo, hi);
+  const int32_t t = lo + (int32_t)(blockIdx.x >> 3);
+  return t < hi ? t : -1;
+}
+
+__device__ inline int32_t tile_select(const TileOne &one, TileArgs &a) {
+  a = one.a;
+  return xcd_tile(one.xcd);
 }
 
 // A grouped launch numbers the tiles of its products consecutively (product j
 // from g.a[j].tile_base); the arguments (kernel-argument memory, read with
 // scalar loads) are those of the product the tile belongs to.
 __device__ inline int32_t tile_select(const TileGroup &g, TileArgs &a) {
-  const int32_t t = xcd_tile(g.total);
+  const int32_t t = xcd_tile(g.xcd);
   if (t < 0) return -1;
   int32_t j = 0;
 #pragma unroll
@@ -693,6 +699,26 @@ __global__ void k_chunk_tile(const int32_t *__restrict__ tchunk, int32_t n_tiles
   const int32_t t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n_tiles) return;
   for (int32_t c = tchunk[t]; c < tchunk[t + 1]; ++c) ctile[c] = t;
+}
+
+// Where each 64th of the work begins, of n launch units with the work w[at[t] *
+// stride] before unit t (at null: w[t]); out[64] = n, then the work of all.
+template <class W>
+__global__ void k_work_parts(const W *__restrict__ w, const int32_t *__restrict__ at, int32_t stride, int32_t n,
+                             int64_t *__restrict__ out) {
+  const int k = threadIdx.x;
+  if (k > cq::kWorkParts) return;
+  auto before = [&](int32_t t) { return (int64_t)w[at ? (int64_t)at[t] * stride : t]; };
+  const int64_t all = before(n);
+  const int64_t want = all / cq::kWorkParts * k + all % cq::kWorkParts * k / cq::kWorkParts;
+  int32_t lo = 0, hi = n;
+  while (lo < hi) {
+    const int32_t mid = lo + (hi - lo) / 2;
+    if (before(mid) < want) lo = mid + 1;
+    else hi = mid;
+  }
+  out[k] = k == cq::kWorkParts ? n : lo;
+  if (k == 0) out[cq::kWorkParts + 1] = all;
 }
 
 // Records of the quadrant kernels, one wavefront per quadrant q (src[q] =
@@ -1592,8 +1618,8 @@ __device__ __forceinline__ void quad_tile(const TileArgs &a, const int32_t tile,
 }
 
 // Global tile number of a launch -> the product's arguments and its tile.
-__device__ inline int32_t tile_at(const TileArgs &arg, int32_t t, TileArgs &a) {
-  a = arg;
+__device__ inline int32_t tile_at(const TileOne &one, int32_t t, TileArgs &a) {
+  a = one.a;
   return t;
 }
 __device__ inline int32_t tile_at(const TileGroup &g, int32_t t, TileArgs &a) {
@@ -1603,26 +1629,20 @@ __device__ inline int32_t tile_at(const TileGroup &g, int32_t t, TileArgs &a) {
   a = g.a[j];
   return t - a.tile_base;
 }
-__device__ inline int32_t total_tiles(const TileArgs &a) { return a.n_tiles; }
-__device__ inline int32_t total_tiles(const TileGroup &g) { return g.total; }
 
-// Persistent launch of class tiles: the grid (a multiple of 8 workgroups, at
-// most one per tile) splits the tiles into 8 contiguous ranges, one per XCD
-// (workgroup b runs on XCD b % 8), and each workgroup takes every (grid/8)-th
-// tile of its XCD's range, so neighbouring tiles (same rows) share an L2.
-// With one workgroup per tile this is the one-tile-per-workgroup order of the
-// other tile kernels.
+// Persistent launch of class tiles: the grid (a multiple of 8 workgroups) gives
+// each XCD (workgroup b runs on XCD b % 8) its tiles, and each workgroup takes
+// every (grid/8)-th of them, so neighbouring tiles (same rows) share an L2. With
+// one workgroup per tile this is the order of the other tile kernels.
 template <int MODE, bool QT, int STG, class ARG>
 __global__ void __launch_bounds__(kTileThreads) k_tile_quad(const ARG arg) {
   using T = typename std::conditional<MODE == 0, double, float>::type;
   constexpr int STAGE = STG + kLdsPad * (int)(8 / sizeof(T));
   __shared__ T stage0[STAGE];
   __shared__ T stage1[STAGE];
-  const int32_t total = total_tiles(arg);
-  const int32_t per = (total + 7) >> 3;
-  const int32_t x = (int32_t)(blockIdx.x & 7), step = (int32_t)(gridDim.x >> 3);
-  const int32_t tend = min(total, (x + 1) * per);
-  for (int32_t tg = x * per + (int32_t)(blockIdx.x >> 3); tg < tend; tg += step) {
+  int32_t tbeg, tend;
+  xcd_units(arg.xcd, tbeg, tend);
+  for (int32_t tg = tbeg + (int32_t)(blockIdx.x >> 3); tg < tend; tg += (int32_t)(gridDim.x >> 3)) {
     __syncthreads();  // the previous tile's last chunk is read before this tile's first copies
     TileArgs a;
     const int32_t tile = tile_at(arg, tg, a);
@@ -1630,11 +1650,18 @@ __global__ void __launch_bounds__(kTileThreads) k_tile_quad(const ARG arg) {
   }
 }
 
+// Workgroups that give every XCD enough for its units.
+unsigned xcd_grid(const int32_t *xcd) {
+  int32_t most = 0;
+  for (int x = 0; x < cq::kXcds; ++x) most = std::max(most, xcd[x + 1] - xcd[x]);
+  return (unsigned)cq::kXcds * (unsigned)most;
+}
+
 template <int MODE, bool QT, class ARG>
-int launch_kind(int kind, const ARG &arg, int32_t n, int32_t wgs, hipStream_t s) {
+int launch_kind(int kind, const ARG &arg, int32_t wgs, hipStream_t s) {
   // One workgroup per tile; the class-tile kernel also runs persistent grids
   // of wgs workgroups (rounded up to a multiple of 8).
-  unsigned gridx = 8u * (unsigned)((n + 7) / 8);
+  unsigned gridx = xcd_grid(arg.xcd);
   if ((kind == kKindQuadSmall || kind == kKindQuadLarge) && wgs > 0)
     gridx = std::min(gridx, 8u * (unsigned)((wgs + 7) / 8));
   const dim3 blk(kTileThreads);
@@ -1654,8 +1681,8 @@ int launch_kind(int kind, const ARG &arg, int32_t n, int32_t wgs, hipStream_t s)
 }
 
 template <int MODE, bool QT, class ARG>
-int launch_uniform(int kind, const ARG &arg, int32_t n, hipStream_t s) {
-  const unsigned gridx = 8u * (unsigned)((n + 7) / 8);
+int launch_uniform(int kind, const ARG &arg, hipStream_t s) {
+  const unsigned gridx = xcd_grid(arg.xcd);
   switch (kind) {
     case kKindUniform + 9: hipLaunchKernelGGL((k_wave_products<MODE, QT, 9, ARG>), dim3(gridx), dim3(64), 0, s, arg); break;
     case kKindUniform + 13: hipLaunchKernelGGL((k_wave_products<MODE, QT, 13, ARG>), dim3(gridx), dim3(64), 0, s, arg); break;
@@ -1666,8 +1693,8 @@ int launch_uniform(int kind, const ARG &arg, int32_t n, hipStream_t s) {
 }
 
 template <int MODE, bool QT, class ARG>
-int launch_quad(int kind, const ARG &arg, int32_t n, int32_t wgs, hipStream_t s) {
-  unsigned gridx = 8u * (unsigned)((n + 7) / 8);
+int launch_quad(int kind, const ARG &arg, int32_t wgs, hipStream_t s) {
+  unsigned gridx = xcd_grid(arg.xcd);
   if (wgs > 0) gridx = std::min(gridx, 8u * (unsigned)((wgs + 7) / 8));
   if (kind == kKindQuadSmall) hipLaunchKernelGGL((k_tile_quad<MODE, QT, kStgSmall, ARG>), dim3(gridx), dim3(kTileThreads), 0, s, arg);
   else hipLaunchKernelGGL((k_tile_quad<MODE, QT, kStgLarge, ARG>), dim3(gridx), dim3(kTileThreads), 0, s, arg);
@@ -1675,26 +1702,26 @@ int launch_quad(int kind, const ARG &arg, int32_t n, int32_t wgs, hipStream_t s)
 }
 
 template <class ARG>
-int launch_any(int mode, bool qt, int kind, const ARG &arg, int32_t n, int32_t wgs, hipStream_t s) {
+int launch_any(int mode, bool qt, int kind, const ARG &arg, int32_t wgs, hipStream_t s) {
   switch (mode * 2 + (qt ? 1 : 0)) {
-    case 0: return launch_kind<0, false, ARG>(kind, arg, n, wgs, s);
-    case 1: return launch_kind<0, true, ARG>(kind, arg, n, wgs, s);
-    case 2: return launch_kind<1, false, ARG>(kind, arg, n, wgs, s);
-    case 3: return launch_kind<1, true, ARG>(kind, arg, n, wgs, s);
-    case 4: return launch_kind<2, false, ARG>(kind, arg, n, wgs, s);
-    case 5: return launch_kind<2, true, ARG>(kind, arg, n, wgs, s);
+    case 0: return launch_kind<0, false, ARG>(kind, arg, wgs, s);
+    case 1: return launch_kind<0, true, ARG>(kind, arg, wgs, s);
+    case 2: return launch_kind<1, false, ARG>(kind, arg, wgs, s);
+    case 3: return launch_kind<1, true, ARG>(kind, arg, wgs, s);
+    case 4: return launch_kind<2, false, ARG>(kind, arg, wgs, s);
+    case 5: return launch_kind<2, true, ARG>(kind, arg, wgs, s);
     // Mode 3 (a block's products of one chunk may be summed in FP32) runs as
     // mode 2, which adds every product in FP64.
-    case 6: return launch_kind<2, false, ARG>(kind, arg, n, wgs, s);
-    case 7: return launch_kind<2, true, ARG>(kind, arg, n, wgs, s);
+    case 6: return launch_kind<2, false, ARG>(kind, arg, wgs, s);
+    case 7: return launch_kind<2, true, ARG>(kind, arg, wgs, s);
     // Split-BF16 x3 (mode 4) runs in the class-tile kernel and the fixed-size
     // kernels of 9x9, 13x13 and 16x16 blocks.
     case 8:
     case 9:
       if (kind == kKindQuadSmall || kind == kKindQuadLarge)
-        return qt ? launch_quad<4, true, ARG>(kind, arg, n, wgs, s) : launch_quad<4, false, ARG>(kind, arg, n, wgs, s);
+        return qt ? launch_quad<4, true, ARG>(kind, arg, wgs, s) : launch_quad<4, false, ARG>(kind, arg, wgs, s);
       if (kind == kKindUniform + 9 || kind == kKindUniform + 13 || kind == kKindUniform + 16)
-        return qt ? launch_uniform<4, true, ARG>(kind, arg, n, s) : launch_uniform<4, false, ARG>(kind, arg, n, s);
+        return qt ? launch_uniform<4, true, ARG>(kind, arg, s) : launch_uniform<4, false, ARG>(kind, arg, s);
       return cq::set_error(CQMM_ERR_STATE, "split-BF16 products need blocks of 9 to 16 or a class-tile schedule");
     default: return cq::set_errorf(CQMM_ERR_ARG, "tile products: precision mode %d", mode);
   }
@@ -1746,6 +1773,7 @@ TileArgs tile_launch_args(const TilePlan &tp, const void *P, const void *Q, void
   a.O = O;
   a.n_tiles = tp.n_wave ? tp.n_wave : tp.n_tiles;
   a.tile_base = 0;
+  a.plan = &tp;
   return a;
 }
 
@@ -1769,13 +1797,20 @@ int tile_group_key(const TilePlan &tp, bool q_trans, int mode) {
 
 int launch_tile_args(const TilePlan &tp, bool q_trans, int mode, const TileArgs &a, hipStream_t s) {
   if (a.n_tiles <= 0) return CQMM_OK;
-  return launch_any(mode, q_trans, tile_kind(tp), a, a.n_tiles, tp.wgs, s);
+  TileOne one;
+  one.a = a;
+  const WorkParts *p = &tp.parts;
+  xcd_split(&p, 1, one.xcd);
+  return launch_any(mode, q_trans, tile_kind(tp), one, tp.wgs, s);
 }
 
-int launch_tile_group(const TilePlan &tp, bool q_trans, int mode, const TileGroup &g, hipStream_t s) {
+int launch_tile_group(const TilePlan &tp, bool q_trans, int mode, TileGroup &g, hipStream_t s) {
   if (g.ngrp <= 0 || g.total <= 0) return CQMM_OK;
   if (g.ngrp > kMaxGroup) return set_errorf(CQMM_ERR_ARG, "grouped tile launch: %d products (at most %d)", g.ngrp, kMaxGroup);
-  return launch_any(mode, q_trans, tile_kind(tp), g, g.total, tp.wgs, s);
+  const WorkParts *p[kMaxGroup];
+  for (int j = 0; j < g.ngrp; ++j) p[j] = &g.a[j].plan->parts;
+  xcd_split(p, g.ngrp, g.xcd);
+  return launch_any(mode, q_trans, tile_kind(tp), g, tp.wgs, s);
 }
 
 // CQMM_TILES=0 builds plans without the tile schedule (triplet kernels only).
@@ -1939,6 +1974,22 @@ int assign_slots(const TileBuildInput &in, const int32_t *tile_out32, DevBuf &d_
   return hip_check(hipStreamSynchronize(s), "slot assignment");
 }
 
+// The plan's work and where its 64ths begin, from the device prefix w (k_work_parts).
+template <class W>
+int work_parts(const W *w, const int32_t *at, int32_t stride, int32_t n, TilePlan &tp, hipStream_t s) {
+  DevBuf d;
+  int64_t h[kWorkParts + 2];
+  int st;
+  if ((st = d.alloc(sizeof(h)))) return st;
+  hipLaunchKernelGGL((k_work_parts<W>), dim3(1), dim3(128), 0, s, w, at, stride, n, d.as<int64_t>());
+  if ((st = hip_check(hipMemcpyAsync(h, d.p, sizeof(h), hipMemcpyDeviceToHost, s), "D2H work parts")) ||
+      (st = hip_check(hipStreamSynchronize(s), "work parts")))
+    return st;
+  for (int k = 0; k <= kWorkParts; ++k) tp.parts.at[k] = (int32_t)h[k];
+  tp.parts.work = h[kWorkParts + 1];
+  return CQMM_OK;
+}
+
 int build_tiles_mixed(const TileBuildInput &in, TilePlan &tp, hipStream_t s);
 
 int build_tiles(const TileBuildInput &in, TilePlan &tp, hipStream_t s) {
@@ -2066,7 +2117,7 @@ int build_tiles(const TileBuildInput &in, TilePlan &tp, hipStream_t s) {
   hipLaunchKernelGGL(fill, grid, dim3(256), 0, s, d_src.as<int32_t>(), tp.n_wave, tp.wave_out.as<int32_t>(), d_tebeg.as<int32_t>(), d_ep.as<int32_t>(), d_eq.as<int32_t>(),
                      nullptr, nullptr, nullptr, tp.pstart.as<int64_t>(), tp.prod.as<uint32_t>());
   if ((st = hip_check(hipGetLastError(), "tile builder launch"))) return st;
-  st = hip_check(hipStreamSynchronize(s), "tile build");
+  st = work_parts(tp.pstart.as<int64_t>(), nullptr, 1, tp.n_wave, tp, s);
   pt.mark("  tiles: entry records");
   return st;
 }
@@ -2265,7 +2316,7 @@ int build_tiles_mixed(const TileBuildInput &in, TilePlan &tp, hipStream_t s) {
     tp.tile_cdim = std::move(d_cdim);
     tp.n_prod = n;
     if ((st = hip_check(hipGetLastError(), "tile builder launch"))) return st;
-    return hip_check(hipStreamSynchronize(s), "tile build");
+    return work_parts(tp.chunk_entry.as<int32_t>(), tp.tile_chunk.as<int32_t>(), 1, tp.n_tiles, tp, s);
   }
   // Product lists.
   DevBuf d_ctile, d_np, d_pbase;
@@ -2303,7 +2354,7 @@ int build_tiles_mixed(const TileBuildInput &in, TilePlan &tp, hipStream_t s) {
                      d_xdim.as<uint8_t>(), nullptr, d_pbase.as<int64_t>(), tp.pstart.as<int64_t>(),
                      tp.pcnt.as<uint64_t>(), tp.prod.as<uint32_t>());
   if ((st = hip_check(hipGetLastError(), "mixed tile builder launch"))) return st;
-  return hip_check(hipStreamSynchronize(s), "mixed tile build");
+  return work_parts(tp.pstart.as<int64_t>(), tp.tile_chunk.as<int32_t>(), kWaves, tp.n_tiles, tp, s);
 }
 
 }  // namespace cq
