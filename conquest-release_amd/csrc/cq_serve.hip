@@ -107,11 +107,13 @@ int64_t cqmm_purify_hbm_estimate(int32_t natoms, int32_t nsf, const cqmm_purify_
   const double t_big = std::max(trip(rL + rS, rL), trip(rL, rL + rS));
   const double trips = trip(rL, rS) + 2 * t_big + trip(rT, rS) + trip(rT, rT) + trip(rT, rH) + trip(rT + rH, rT);
   // Resident triplet lists and tile schedules (14 B per product) + the largest
-  // build's transient buffers (38 B per product of the biggest product). The
-  // coefficients are fitted to the measured per-solve peaks (hbm_peak) of
-  // 64-2048 atoms with 4 and 13 support functions, where this sum (x1.1) is
-  // 1.18-1.68 times the peak.
-  const double plans = 14.0 * trips + 38.0 * t_big;
+  // build's transient buffers (38 B per product of the biggest product); blocks
+  // below 4x4 have few products per entry of their schedule, so more bytes for each
+  // (20 and 50). Fitted to the measured per-solve peaks (hbm_peak): this sum (x1.1)
+  // is 1.21-1.93 times the peak at 8/8/12 A, 64-2048 atoms with 4 and 13 support
+  // functions, and at least 1.05 times it for 1 to 17 at 3/3/9 to 6/6/16 A.
+  const double per = nsf < 4 ? 20.0 : 14.0, per_build = nsf < 4 ? 50.0 : 38.0;
+  const double plans = per * trips + per_build * t_big;
   return (int64_t)(1.1 * (mats + f32 + plans)) + (64LL << 20);
 }
 
