@@ -60,32 +60,29 @@ struct DevBuf {
   template <class T> T *as() const { return static_cast<T *>(p); }
 };
 
-// Output-tile schedule of one product with a uniform block size (NSF x NSF
-// blocks stored contiguously, so every offset is a multiple of NSF^2 and is kept
-// as a block index). A tile is kTileRows primary atoms x kTileCols column atoms
-// of the output; its entries are the contraction atoms x with at least one
-// product in the tile, each carrying which of the tile's left-operand blocks
-// (row, x) and right-operand blocks (column, x) exist. Entries are grouped into
-// chunks whose operand blocks fit the kernel's LDS stage.
+// Output-tile schedule of one product. A tile is kTileRows primary atoms x
+// kTileCols column atoms of the output; its entries are the contraction atoms x
+// with at least one product in the tile, each with those of the tile's
+// left-operand blocks (row, x) and right-operand blocks (column, x) that exist.
 constexpr int kTileRows = 8, kTileCols = 8;
 struct TilePlan {
   int nsf = 0;
   int32_t n_tiles = 0, n_chunks = 0;
   int64_t n_entries = 0, n_loads = 0, n_prod = 0;
+  // Uniform sizes (k_wave_products; 4x4 blocks, dense: k_quad4; blocks of NSF x
+  // NSF stored contiguously, kept by block index): the 4x4-block quadrants of the
+  // tiles that hold an output block, each the work of one wavefront. pstart is
+  // then int64 [n_wave+1], the first record word of each quadrant, prod uint32 the
+  // record words, with padding.
+  int32_t n_wave = 0;
+  DevBuf wave_out;     // int32 [n_wave*16] output block row * 4 + column of each quadrant, or -1
+  // Mixed sizes: entries are grouped into chunks whose operand blocks fit the
+  // kernel's LDS stage.
   DevBuf tile_chunk;   // int32 [n_tiles+1]  first chunk of each tile
-  DevBuf chunk_lbeg;   // int64 [n_chunks+1] first operand of each chunk in `list`
-  DevBuf list;         // int32 [n_loads] operand block index; bit 31 set: right operand
+  DevBuf chunk_lbeg;   // int64 [n_chunks+1] first operand of each chunk in `list64`
   DevBuf pstart;       // int64 [(n_chunks+1)*4] first product of (chunk, wavefront) in `prod`
   DevBuf pcnt;         // uint64 [(n_chunks+1)*4] products of (chunk, wavefront) per slot, 4 bits each
-  DevBuf prod;         // uint32 [n_prod+64] LDS element offsets of the two operands (left | right << 16)
-  DevBuf tile_out;     // int32 [n_tiles*64] output block of slot row*8+col, or -1
-  DevBuf wave_out;     // int32 [n_tiles*4*16] output block of (tile, wavefront, slot), or -1
-  // Uniform sizes (k_wave_products; 4x4 blocks, dense: k_quad4): the 4x4-block
-  // quadrants of the tiles that hold an output block, each the work of one
-  // wavefront. wave_out is then [n_wave*16] (row * 4 + column within the
-  // quadrant), pstart [n_wave+1] the first record word of each quadrant and prod
-  // the record words, with padding.
-  int32_t n_wave = 0;
+  DevBuf prod;         // uint32 [n_prod+64] product words (k_chunk_prods_mx)
   // Mixed sizes up to 4x4 (dense): each wavefront computes a 4x4-block quadrant
   // of the tile per entry with one MFMA; no product lists.
   bool dense = false;
@@ -98,7 +95,7 @@ struct TilePlan {
   DevBuf tile_rdim;    // uint8 [n_tiles*8] rows of each tile row's blocks (mixed dense: blocks up to 4x4)
   DevBuf tile_cdim;    // uint8 [n_tiles*8] columns of each tile column's blocks
   // Mixed block sizes (maxn > 0): operands and outputs by element offset.
-  int maxn = 0;        // largest block dimension; 0: uniform schedule above
+  int maxn = 0;        // largest block dimension; 0: uniform sizes
   DevBuf list64;       // uint64 [n_loads] operand element offset; bit 63 set: right operand
   DevBuf listls;       // uint32 [n_loads] LDS element offset in the chunk | elements << 16
   DevBuf wave_out64;   // int64 [n_tiles*4*16] output element offset of (tile, wavefront, slot), or -1
@@ -111,7 +108,6 @@ struct TilePlan {
 struct TileArgs {
   const int32_t *tile_chunk;
   const int64_t *chunk_lbeg;
-  const int32_t *list;          // uniform sizes: operand block indices
   const uint64_t *list64;       // mixed sizes: operand element offsets
   const uint32_t *listls;       // mixed sizes: LDS offsets and sizes
   const int64_t *pstart;

@@ -905,7 +905,8 @@ __global__ void k_list_fill_mx(const int64_t *__restrict__ ep, const int64_t *__
 }
 
 // Chunks of a tile by operand elements (at most cap), entries, operand
-// blocks (at most kWaves * 64) and wavefront products (as k_chunks).
+// blocks (at most kWaves * 64) and products per wavefront (kWaveProducts). Count
+// pass (FILL unset): chunks of each tile. Fill pass: each chunk's first entry.
 template <bool FILL>
 __global__ void k_chunks_mx(const int32_t *__restrict__ tebeg, const uint32_t *__restrict__ mask,
                             const int32_t *__restrict__ esz, const uint8_t *__restrict__ owner, int32_t n_tiles,
@@ -968,8 +969,10 @@ __global__ void k_list_lds_mx(const int64_t *__restrict__ chunk_lbeg, const uint
   }
 }
 
-// Product lists (as k_chunk_prods): word = left LDS offset | right LDS offset
-// << 12 | (contraction dimension nx - 1) << 24 | (k-steps - 1) << 28 |
+// Product lists of each chunk, sorted by (wavefront, slot, entry). Count pass (FILL
+// unset): products per chunk into np. Fill pass, with pbase = the chunk's first
+// product: pstart and pcnt of its wavefronts, and the product words. Word = left
+// LDS offset | right LDS offset << 12 | (contraction dimension nx - 1) << 24 | (k-steps - 1) << 28 |
 // (contraction indices of the last k-step - 1) << 30.
 template <bool FILL>
 __global__ void k_chunk_prods_mx(int32_t nch, const int32_t *__restrict__ chunk_entry,
@@ -1754,7 +1757,6 @@ TileArgs tile_launch_args(const TilePlan &tp, const void *P, const void *Q, void
   std::memset(&a, 0, sizeof(a));
   a.tile_chunk = tp.tile_chunk.as<int32_t>();
   a.chunk_lbeg = tp.chunk_lbeg.as<int64_t>();
-  a.list = tp.list.as<int32_t>();
   a.list64 = tp.list64.as<uint64_t>();
   a.listls = tp.listls.as<uint32_t>();
   a.pstart = tp.pstart.as<int64_t>();
@@ -2001,25 +2003,17 @@ int build_tiles(const TileBuildInput &in, TilePlan &tp, hipStream_t s) {
   tp = TilePlan();
   tp.nsf = in.nsf;
   tp.n_tiles = in.n_tiles;
-  // Output blocks by block index (element offset / NSF^2).
-  std::vector<int32_t> tout32((size_t)in.n_tiles * 64);
-  parallel_for((int64_t)tout32.size(), [&](int64_t b, int64_t e) {
-    for (int64_t k = b; k < e; ++k) tout32[k] = in.tile_out[k] < 0 ? -1 : (int32_t)(in.tile_out[k] / ns2);
-  });
-  if ((st = tp.tile_out.alloc((size_t)in.n_tiles * 64 * 4))) return st;
-  if ((st = hip_check(hipMemcpyAsync(tp.tile_out.p, tout32.data(), (size_t)in.n_tiles * 64 * 4, hipMemcpyHostToDevice, s),
-                      "H2D tile_out")) ||
-      (st = hip_check(hipStreamSynchronize(s), "tile_out")))
-    return st;
   tp.dense = in.nsf == kDenseNsf;
-  // Output blocks of the tiles' quadrants: quadrant (w / 2, w % 2) has rows
-  // 4*(w/2)..+3, columns 4*(w%2)..+3.
+  // Output blocks of the tiles' quadrants by block index (element offset /
+  // NSF^2): quadrant (w / 2, w % 2) has rows 4*(w/2)..+3, columns 4*(w%2)..+3.
   std::vector<int32_t> wave_out((size_t)in.n_tiles * 64, -1), src;
   parallel_for(in.n_tiles, [&](int64_t b, int64_t e) {
     for (int64_t t = b; t < e; ++t)
       for (int u = 0; u < 8; ++u)
-        for (int c = 0; c < 8; ++c)
-          wave_out[(t * kWaves + (u >> 2) * 2 + (c >> 2)) * 16 + (u & 3) * 4 + (c & 3)] = tout32[t * 64 + u * 8 + c];
+        for (int c = 0; c < 8; ++c) {
+          const int64_t o = in.tile_out[t * 64 + u * 8 + c];
+          if (o >= 0) wave_out[(t * kWaves + (u >> 2) * 2 + (c >> 2)) * 16 + (u & 3) * 4 + (c & 3)] = (int32_t)(o / ns2);
+        }
   });
   // Only the quadrants with output blocks are work.
   src.reserve((size_t)in.n_tiles * kWaves);
