@@ -603,6 +603,38 @@ __global__ void __launch_bounds__(64) k_quad4(const ARG arg) {
   // FP64 accumulator D[g+4e][r], FP32 D[4g+e][r]: quadrant row R, column r is
   // element (R % 4, r % 4) of block (R / 4, r / 4).
   const int32_t *wo = a.wave_out + (int64_t)tile * 16;
+  // The matrix step also multiplies the zeros of an absent block by the other
+  // operand, which is NaN where that is infinite or NaN. A NaN is therefore
+  // summed again from the products that exist (no cost without one).
+  bool nan = false;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) nan |= MODE == 1 ? a32[e] != a32[e] : a64[e] != a64[e];
+  if (__ballot(nan) != 0) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (MODE == 1 ? a32[e] == a32[e] : a64[e] == a64[e]) continue;
+      const int rq = MODE == 0 ? e : g, ri = MODE == 0 ? g : e;
+      const uint32_t *rec = a.prod + w0;
+      double sum = 0.0;
+      float sum32 = 0.f;
+      for (int32_t i = 0; i < n; ++i, rec += 8) {
+        const uint32_t bp = rec[rq], bq = rec[4 + (r >> 2)];
+        if (bp == ~0u || bq == ~0u) continue;
+        const T *x = static_cast<const T *>(a.P) + (int64_t)bp * 16 + ri;
+        const T *y = static_cast<const T *>(a.Q) + (int64_t)bq * 16 + (QT ? r & 3 : 4 * (r & 3));
+        float part = MODE == 1 ? sum32 : 0.f;
+        for (int k = 0; k < 4; ++k) {
+          const T xk = x[4 * k], yk = y[QT ? 4 * k : k];
+          if constexpr (MODE == 0) sum = __builtin_fma(xk, yk, sum);
+          else part = __builtin_fmaf(xk, yk, part);
+        }
+        if constexpr (MODE == 1) sum32 = part;
+        if constexpr (MODE == 2) sum += (double)part;
+      }
+      if constexpr (MODE == 1) a32[e] = sum32;
+      else a64[e] = sum;
+    }
+  }
   auto write = [&](auto *out) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
