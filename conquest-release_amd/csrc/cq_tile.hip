@@ -1405,6 +1405,41 @@ __global__ void __launch_bounds__(kTileThreads) k_tile_dense_mx(
   // Quadrant row R, column r: element (R % 4, r % 4) of block (R / 4, r / 4);
   // written where it lies inside that block's shape.
   const int64_t *wo = wave_out + ((int64_t)tile * kWaves + w) * 16;
+  // As in k_quad4, a NaN is summed again from the products that exist.
+  bool nan = false;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) nan |= MODE == 1 ? a32[e] != a32[e] : a64[e] != a64[e];
+  if (__ballot(nan) != 0) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (MODE == 1 ? a32[e] == a32[e] : a64[e] == a64[e]) continue;
+      const int u = 4 * qr + (MODE == 0 ? e : g), ri = MODE == 0 ? g : e;
+      const int nr = rdim[(int64_t)tile * 8 + u];
+      if (ri >= nr || rr >= cd) continue;
+      double sum = 0.0;
+      float sum32 = 0.f;
+      int64_t at = chunk_lbeg[c0];
+      for (int32_t i = chunk_entry[c0]; i < chunk_entry[c1]; ++i) {
+        const uint32_t m = emask[i], ym = m & 0xffu, bm = (m >> 8) & 0xffu;
+        if ((ym >> u & 1u) && (bm >> cb & 1u)) {
+          const int nx = (int)((m >> 16) & 15u) + 1;
+          const T *x = P + list64[at + __popc(ym & ((1u << u) - 1u))] + ri;
+          const T *y = Q + (list64[at + __popc(ym) + __popc(bm & below_b)] & ~(1ull << 63)) + (QT ? rr : nx * rr);
+          float part = MODE == 1 ? sum32 : 0.f;
+          for (int k = 0; k < nx; ++k) {
+            const T xk = x[nr * k], yk = y[QT ? cd * k : k];
+            if constexpr (MODE == 0) sum = __builtin_fma(xk, yk, sum);
+            else part = __builtin_fmaf(xk, yk, part);
+          }
+          if constexpr (MODE == 1) sum32 = part;
+          if constexpr (MODE == 2) sum += (double)part;
+        }
+        at += __popc(m & 0xffffu);
+      }
+      if constexpr (MODE == 1) a32[e] = sum32;
+      else a64[e] = sum;
+    }
+  }
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int rq = MODE == 0 ? e : g, ri = MODE == 0 ? g : e;

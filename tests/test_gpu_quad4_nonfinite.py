@@ -1,9 +1,8 @@
-"""GPU test: in products of 4x4 blocks infinities and NaNs reach exactly the
+"""GPU test: in products of blocks up to 4x4 infinities and NaNs reach exactly the
 results that use them.
 
-One 4x4 matrix step covers 16 block pairs, those with an absent block as zeros.
-Blocks of both operands get an infinity and a NaN; the results' non-finite
-elements and infinities must be the oracle's, and the finite ones within the
+One matrix step covers 16 block pairs, those with an absent block as zeros. Both
+operands get infinities and NaNs; the results' non-finite elements and infinities must be the oracle's, and the finite ones within the
 bars of the mode: 1e-12 (FP64, a few thousand terms of 1.1e-16), 2e-5 and 2e-6
 (FP32 operands, FP32 and FP64 sums: 6e-8 per operand and term).
 """
@@ -21,16 +20,19 @@ pytestmark = pytest.mark.gpu
                                        (cqmm.CQMM_FP32 | cqmm.CQMM_FP32_ACC64, 2e-6)])
 @pytest.mark.parametrize("natoms,ra,rb,rc", [(1, 4.0, 5.0, 3.0), (41, 6.0, 7.0, 9.0), (27, 13.0, 13.0, 13.0),
                                              (60, 5.0, 5.0, 10.0)])
+@pytest.mark.parametrize("nsf", [4, 3, ((4, .6), (1, .4))])
 @pytest.mark.parametrize("mt", [1, 2])
-def test_nonfinite_values_stay_in_their_products(mt, natoms, ra, rb, rc, flags, bar):
-    case = Case(natoms, 4, ra, rb, rc, mt, seed=19)
+def test_nonfinite_values_stay_in_their_products(mt, nsf, natoms, ra, rb, rc, flags, bar):
+    case = Case(natoms, nsf, ra, rb, rc, mt, seed=19)
     plan = cqmm.Plan(case.desc)
+    sizes = set(case.nsf.tolist())
+    assert plan.info().tile_family == (cqmm.TILES_DENSE4 if sizes == {4} else cqmm.TILES_DENSE_MIXED)
     a, b, c = case.values()
-    left = (a if mt == 1 else c).reshape(-1, 16)
-    right = b.reshape(-1, 16)
-    left[min(3, len(left) - 1), 5] = np.inf
-    left[len(left) // 2, [0, 15]] = np.nan, -np.inf
-    right[len(right) // 3, 7] = np.inf
+    left = a if mt == 1 else c
+    left[min(50, len(left) - 1)] = np.inf
+    left[len(left) // 2] = np.nan
+    left[len(left) * 3 // 4] = -np.inf
+    b[len(b) // 3] = np.inf
     x, y, z = a.copy(), b.copy(), c.copy()
     with np.errstate(invalid="ignore"):
         oracle.mat_mult(case.desc, x, y, z)
