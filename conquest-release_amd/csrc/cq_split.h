@@ -9,7 +9,7 @@ namespace cq {
 constexpr int kXcds = 8;
 constexpr int kWorkParts = 64;
 
-// Work of one product's launch units (record words, products or entries) and the
+// Work of one product's launch units (record words, k-steps or entries) and the
 // units where each 64th of it begins; at[64] = the number of units.
 struct WorkParts {
   int64_t work = 0;

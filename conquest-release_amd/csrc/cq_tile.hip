@@ -733,14 +733,14 @@ __global__ void k_chunk_tile(const int32_t *__restrict__ tchunk, int32_t n_tiles
   for (int32_t c = tchunk[t]; c < tchunk[t + 1]; ++c) ctile[c] = t;
 }
 
-// Where each 64th of the work begins, of n launch units with the work w[at[t] *
-// stride] before unit t (at null: w[t]); out[64] = n, then the work of all.
+// Where each 64th of the work begins, of n launch units with the work w[at[t]]
+// before unit t (at null: w[t]); out[64] = n, then the work of all.
 template <class W>
-__global__ void k_work_parts(const W *__restrict__ w, const int32_t *__restrict__ at, int32_t stride, int32_t n,
+__global__ void k_work_parts(const W *__restrict__ w, const int32_t *__restrict__ at, int32_t n,
                              int64_t *__restrict__ out) {
   const int k = threadIdx.x;
   if (k > cq::kWorkParts) return;
-  auto before = [&](int32_t t) { return (int64_t)w[at ? (int64_t)at[t] * stride : t]; };
+  auto before = [&](int32_t t) { return (int64_t)w[at ? at[t] : t]; };
   const int64_t all = before(n);
   const int64_t want = all / cq::kWorkParts * k + all % cq::kWorkParts * k / cq::kWorkParts;
   int32_t lo = 0, hi = n;
@@ -1001,8 +1001,13 @@ __global__ void k_list_lds_mx(const int64_t *__restrict__ chunk_lbeg, const uint
   }
 }
 
+// Work of a chunk in the mixed-size kernel for the split over the XCDs, in parts of
+// a k-step: three per product beside its k-steps, 100 for the chunk (its barrier and
+// copies). With products alone the 4096-atom 4/9/13 mix takes 27.0 to 27.2 ms, so 26.8.
+constexpr int kWorkProduct = 3, kWorkChunk = 100;
+
 // Product lists of each chunk, sorted by (wavefront, slot, entry). Count pass (FILL
-// unset): products per chunk into np. Fill pass, with pbase = the chunk's first
+// unset): products per chunk into np, its work into `work`. Fill pass, with pbase = the chunk's first
 // product: pstart and pcnt of its wavefronts, and the product words. Word = left
 // LDS offset | right LDS offset << 12 | (contraction dimension nx - 1) << 24 | (k-steps - 1) << 28 |
 // (contraction indices of the last k-step - 1) << 30.
@@ -1012,9 +1017,9 @@ __global__ void k_chunk_prods_mx(int32_t nch, const int32_t *__restrict__ chunk_
                                  const int32_t *__restrict__ coff, const int32_t *__restrict__ ex,
                                  const uint8_t *__restrict__ owner, const uint8_t *__restrict__ rdim,
                                  const uint8_t *__restrict__ cdim, const uint8_t *__restrict__ xdim,
-                                 int64_t *__restrict__ np, const int64_t *__restrict__ pbase,
-                                 int64_t *__restrict__ pstart, uint64_t *__restrict__ pcnt,
-                                 uint32_t *__restrict__ prod) {
+                                 int64_t *__restrict__ np, int64_t *__restrict__ work,
+                                 const int64_t *__restrict__ pbase, int64_t *__restrict__ pstart,
+                                 uint64_t *__restrict__ pcnt, uint32_t *__restrict__ prod) {
   const int32_t c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= nch) return;
   const int64_t t = ctile[c];
@@ -1022,9 +1027,10 @@ __global__ void k_chunk_prods_mx(int32_t nch, const int32_t *__restrict__ chunk_
   const int32_t e0 = chunk_entry[c], e1 = chunk_entry[c + 1];
   uint8_t cnt[64];
   for (int i = 0; i < 64; ++i) cnt[i] = 0;
-  int32_t tot = 0;
+  int32_t tot = 0, steps = 0;
   for (int32_t e = e0; e < e1; ++e) {
     const uint32_t m = mask[e];
+    const int32_t before = tot;
     for (uint32_t ym = m & 0xffu; ym; ym &= ym - 1u) {
       const int u = __builtin_ctz(ym);
       for (uint32_t bm = (m >> 8) & 0xffu; bm; bm &= bm - 1u) {
@@ -1035,9 +1041,11 @@ __global__ void k_chunk_prods_mx(int32_t nch, const int32_t *__restrict__ chunk_
         }
       }
     }
+    steps += (tot - before) * ((xdim[ex[e]] + 3) >> 2);
   }
   if (!FILL) {
     np[c] = tot;
+    work[c] = kWorkProduct * tot + steps + kWorkChunk;
     return;
   }
   uint16_t off[64];
@@ -2045,12 +2053,12 @@ int assign_slots(const TileBuildInput &in, const int32_t *tile_out32, DevBuf &d_
 
 // The plan's work and where its 64ths begin, from the device prefix w (k_work_parts).
 template <class W>
-int work_parts(const W *w, const int32_t *at, int32_t stride, int32_t n, TilePlan &tp, hipStream_t s) {
+int work_parts(const W *w, const int32_t *at, int32_t n, TilePlan &tp, hipStream_t s) {
   DevBuf d;
   int64_t h[kWorkParts + 2];
   int st;
   if ((st = d.alloc(sizeof(h)))) return st;
-  hipLaunchKernelGGL((k_work_parts<W>), dim3(1), dim3(128), 0, s, w, at, stride, n, d.as<int64_t>());
+  hipLaunchKernelGGL((k_work_parts<W>), dim3(1), dim3(128), 0, s, w, at, n, d.as<int64_t>());
   if ((st = hip_check(hipMemcpyAsync(h, d.p, sizeof(h), hipMemcpyDeviceToHost, s), "D2H work parts")) ||
       (st = hip_check(hipStreamSynchronize(s), "work parts")))
     return st;
@@ -2178,7 +2186,7 @@ int build_tiles(const TileBuildInput &in, TilePlan &tp, hipStream_t s) {
   hipLaunchKernelGGL(fill, grid, dim3(256), 0, s, d_src.as<int32_t>(), tp.n_wave, tp.wave_out.as<int32_t>(), d_tebeg.as<int32_t>(), d_ep.as<int32_t>(), d_eq.as<int32_t>(),
                      nullptr, nullptr, nullptr, tp.pstart.as<int64_t>(), tp.prod.as<uint32_t>());
   if ((st = hip_check(hipGetLastError(), "tile builder launch"))) return st;
-  st = work_parts(tp.pstart.as<int64_t>(), nullptr, 1, tp.n_wave, tp, s);
+  st = work_parts(tp.pstart.as<int64_t>(), nullptr, tp.n_wave, tp, s);
   pt.mark("  tiles: entry records");
   return st;
 }
@@ -2377,21 +2385,24 @@ int build_tiles_mixed(const TileBuildInput &in, TilePlan &tp, hipStream_t s) {
     tp.tile_cdim = std::move(d_cdim);
     tp.n_prod = n;
     if ((st = hip_check(hipGetLastError(), "tile builder launch"))) return st;
-    return work_parts(tp.chunk_entry.as<int32_t>(), tp.tile_chunk.as<int32_t>(), 1, tp.n_tiles, tp, s);
+    return work_parts(tp.chunk_entry.as<int32_t>(), tp.tile_chunk.as<int32_t>(), tp.n_tiles, tp, s);
   }
   // Product lists.
-  DevBuf d_ctile, d_np, d_pbase;
+  DevBuf d_ctile, d_np, d_pbase, d_work;
   if ((st = d_ctile.alloc((size_t)std::max(nch, 1) * 4)) || (st = d_np.alloc((size_t)std::max(nch, 1) * 8)) ||
-      (st = d_pbase.alloc(((size_t)nch + 1) * 8)))
+      (st = d_pbase.alloc(((size_t)nch + 1) * 8)) || (st = d_work.alloc(((size_t)nch + 1) * 8)))
     return st;
   hipLaunchKernelGGL(k_chunk_tile, dim3(grid1(in.n_tiles, 256)), dim3(256), 0, s, tp.tile_chunk.as<int32_t>(),
                      in.n_tiles, d_ctile.as<int32_t>());
   hipLaunchKernelGGL((k_chunk_prods_mx<false>), dim3(grid1(std::max(nch, 1), 256)), dim3(256), 0, s, nch,
                      d_centry.as<int32_t>(), d_ctile.as<int32_t>(), d_emask.as<uint32_t>(), d_ecoff.as<int32_t>(),
                      d_ex.as<int32_t>(), d_owner.as<uint8_t>(), d_rdim.as<uint8_t>(), d_cdim.as<uint8_t>(),
-                     d_xdim.as<uint8_t>(), d_np.as<int64_t>(), nullptr, nullptr, nullptr, nullptr);
+                     d_xdim.as<uint8_t>(), d_np.as<int64_t>(), d_work.as<int64_t>() + 1, nullptr, nullptr, nullptr,
+                     nullptr);
   if ((st = hip_check(hipMemsetAsync(d_pbase.p, 0, 8, s), "memset pbase"))) return st;
   if ((st = inclusive_scan(d_np.as<int64_t>(), d_pbase.as<int64_t>() + 1, (size_t)nch, s))) return st;
+  if ((st = hip_check(hipMemsetAsync(d_work.p, 0, 8, s), "memset work"))) return st;
+  if ((st = inclusive_scan(d_work.as<int64_t>() + 1, d_work.as<int64_t>() + 1, (size_t)nch, s))) return st;
   int64_t nprod = 0;
   if ((st = hip_check(hipMemcpyAsync(&nprod, d_pbase.as<int64_t>() + nch, 8, hipMemcpyDeviceToHost, s), "D2H products")) ||
       (st = hip_check(hipStreamSynchronize(s), "product count")))
@@ -2412,10 +2423,10 @@ int build_tiles_mixed(const TileBuildInput &in, TilePlan &tp, hipStream_t s) {
   hipLaunchKernelGGL((k_chunk_prods_mx<true>), dim3(grid1(std::max(nch, 1), 256)), dim3(256), 0, s, nch,
                      d_centry.as<int32_t>(), d_ctile.as<int32_t>(), d_emask.as<uint32_t>(), d_ecoff.as<int32_t>(),
                      d_ex.as<int32_t>(), d_owner.as<uint8_t>(), d_rdim.as<uint8_t>(), d_cdim.as<uint8_t>(),
-                     d_xdim.as<uint8_t>(), nullptr, d_pbase.as<int64_t>(), tp.pstart.as<int64_t>(),
+                     d_xdim.as<uint8_t>(), nullptr, nullptr, d_pbase.as<int64_t>(), tp.pstart.as<int64_t>(),
                      tp.pcnt.as<uint64_t>(), tp.prod.as<uint32_t>());
   if ((st = hip_check(hipGetLastError(), "mixed tile builder launch"))) return st;
-  return work_parts(tp.pstart.as<int64_t>(), tp.tile_chunk.as<int32_t>(), kWaves, tp.n_tiles, tp, s);
+  return work_parts(d_work.as<int64_t>(), tp.tile_chunk.as<int32_t>(), tp.n_tiles, tp, s);
 }
 
 }  // namespace cq
