@@ -201,9 +201,8 @@ def multiply_workload(name, args, fp32_modes=True, cpu=False):
                 algorithmic_bytes=algo_bytes, tflops_fp64=round(flops / (kern_avg_ms / 1e3) / 1e12, 3))
     # The same products with FP32 MFMA on FP32 copies of the operands (per call:
     # FP64->FP32 operand copies, products, FP32->FP64 result): FP32 accumulation
-    # (CQMM_FP32), each product's FP32 result summed in FP64 (CQMM_FP32_ACC64), and
-    # a block's products summed in FP32 within a chunk, chunks in FP64
-    # (CQMM_FP32_RUN64); errors against the FP64 result.
+    # (CQMM_FP32), each product's FP32 result summed in FP64 (CQMM_FP32_ACC64, and
+    # CQMM_FP32_RUN64, which runs as it); errors against the FP64 result.
     fp32 = {}
     modes = (("fp32_accumulate", 0), ("fp32_acc64", cqmm.CQMM_FP32_ACC64), ("fp32_run64", cqmm.CQMM_FP32_RUN64))
     if info.kernel == cqmm.KERNEL_TILE and info.tile_family in (cqmm.TILES_CLASS, cqmm.TILES_UNIFORM + 9,

@@ -157,7 +157,7 @@ struct TripletPlan {
   DevBuf seg_mn;            // uint8 [2*n_seg] (non-uniform only)
   DevBuf tp, tq;            // int32 or int64 [n_trip]
   DevBuf tk;                // uint8 [n_trip] inner dimension (non-uniform only)
-  TilePlan tiles;           // FP64 tile schedule (uniform block sizes), n_tiles == 0 if absent
+  TilePlan tiles;           // tile schedule (blocks up to 16), n_tiles == 0 if absent
   int kernel = 0;           // CQMM_KERNEL_* selection for the FP64 path
   // Symmetric results (cqmm_plan_create_symmetric): of each transpose pair of
   // result blocks (p, q), p < q, only p is computed; the launchers then write
@@ -192,7 +192,7 @@ bool class_tiles_enabled();
 bool morton_rows_enabled();
 bool primary_rows_forced();
 // Uniform 9, 13, 16 blocks as one class of the class-tile schedule
-// (CQMM_UNIFORM_TILES=class; default: the fixed-size tile kernel).
+// (CQMM_UNIFORM_TILES=class; default: the wavefront kernel).
 bool uniform_class_tiles_enabled();
 // Ranks of n items in the order (size[i], rank[i]), each size group starting
 // at a multiple of 8.

@@ -614,8 +614,8 @@ int build_plan(const DescV<H> *d, cqmm_plan **out) {
   if (n_trip > INT32_MAX) return cq::set_error(CQMM_ERR_RANGE, "cqmm_plan_create: more than 2^31 block products");
 
   // ---- output tiles: host part ----
-  // Uniform instanced sizes take the fixed-size tile kernel; other sizes up to
-  // 16 (mixed species) the mixed-size one.
+  // Uniform 4, 9, 13 and 16 take the wavefront kernels over the tiles' quadrants;
+  // other sizes up to 16 (mixed species) the mixed-size tile kernel.
   bool tiles = (uniform != 0 || (maxn > 0 && maxn <= 16)) && n_trip > 0 && cq::tiles_enabled();
   const int64_t ns2 = (int64_t)uniform * uniform;
   std::vector<int32_t> crank, tmap, rrank;  // rrank: tile row rank of each primary atom (empty: primary order)
@@ -625,7 +625,7 @@ int build_plan(const DescV<H> *d, cqmm_plan **out) {
   bool class_uniform = false;
   const int64_t nx = d->mult_type == 1 ? ni_a : ni_c;
   // Uniform 9, 13 and 16 may run as one class of the class-tile schedule
-  // (CQMM_UNIFORM_TILES=class) instead of the fixed-size tile kernel.
+  // (CQMM_UNIFORM_TILES=class) instead of the wavefront kernel.
   const bool uclass = uniform != 0 && uniform != 4 && cq::uniform_class_tiles_enabled();
   if (tiles && uniform && !uclass) {
     // Every operand offset must be a whole number of blocks.

@@ -296,16 +296,19 @@ __device__ inline void wait_blocks(int32_t after) {
 // What bounds it (gfx950): a VALU instruction holds the SIMD as a matrix
 // instruction does (3 f64 MFMA take 217 cycles, with 16 VALU instructions of any
 // wavefront between them 292), so a product costs its matrix steps plus 4.6
-// cycles per VALU instruction, and the design keeps these few; what is left
-// is the scalar work and the branches of a record (about 1500 cycles of one
-// wavefront) and, at thousands of atoms, the copies beyond L2 (4096 atoms 13x13,
-// type 2: copies alone 34.5 ms, everything but the copies 37.5 ms).
+// cycles per VALU instruction, and the design keeps these few. What is left
+// is the scalar work and the branches of a record (4096 atoms 13x13, type 2: 31
+// scalar instructions and 7 branches per product against 3 matrix steps and 7
+// other VALU instructions, the matrix cores busy 48%) and, at thousands of
+// atoms, the copies beyond L2 (copies alone 34.5 ms, everything else 37.5 ms).
 // Against one workgroup per 8x8 tile with its four wavefronts in step (a barrier
 // per chunk; the busiest wavefront has 1.25 to 1.56 times the mean products):
-// 13x13 FP64 4096 atoms type 2 50.2 -> 46.0 ms, 1024 atoms symmetric
-// 15.9 -> 15.3 ms, 9x9 FP32 with FP64 sums 1500 atoms 11.1 -> 8.9 ms, 13x13 split
-// BF16 1024 atoms 5.9 -> 5.0 ms (4.2 ms with the FP64 result written here, not
-// widened by a pass of its own), 9x9 FP64 60 atoms (one LNV solve) 12.5 -> 10.0 ms.
+// 13x13 FP64 4096 atoms type 2 50.6 -> 44.8 ms, 1024 atoms symmetric
+// 15.8 -> 13.15 ms, 9x9 FP32 with FP64 sums 1500 atoms 11.0 -> 8.74 ms, 13x13 split
+// BF16 1024 atoms 5.92 -> 4.02 ms (0.8 of it the FP64 result written here, not
+// widened by a pass of its own), 9x9 FP64 2000 atoms 8/12/16 A 9.97 -> 7.80 ms, 16x16 FP64
+// 1500 atoms 8/12/16 A 29.3 -> 14.2 ms, type 2 12/12/8 A 10.0 -> 7.73 ms, one LNV
+// evaluation of 60 atoms 9x9 12.4 -> 9.6 ms.
 // Tried and slower: operands straight to registers (4096 atoms 58 ms: 18 to 33
 // address cycles per load), two stages instead of the ring (split BF16 6.2 ms),
 // three wavefronts per SIMD with right operands read per product (9x9 11.1 ms).
@@ -524,11 +527,11 @@ k_wave_products(const ARG arg) {
 //
 // What bounds it: a record takes one 72-cycle f64 matrix step and about ten VALU
 // instructions, and copies from L2 (13 to 16 TB/s) what its products read: 512
-// atoms, 2.0e7 products, 0.215 ms. One workgroup per 8x8 tile with a barrier per
+// atoms, 2.0e7 products, 0.21 ms. One workgroup per 8x8 tile with a barrier per
 // chunk took 0.80 ms; a list of products per output block with v_mfma_f64_4x4x4
 // (four output blocks to a wavefront) 0.45 ms, as it copies 2 blocks per product
 // and not the 0.6 to 0.9 of a record. One McWeeny batch of 4 x 64 atoms
-// 73.7 -> 26.9 ms.
+// 73.7 -> 26.8 ms.
 __device__ __attribute__((aligned(128))) uint32_t g_zero_block[32];
 
 template <int MODE, bool QT, class ARG>
