@@ -23,8 +23,21 @@ struct WorkParts {
 // units each / runs of 8192 / equal work: 13x13 1024 atoms symmetric 15.8 / 13.5
 // / 13.1 ms, 4/9/13 mixes of 4096 atoms 27.5 / 26.8 / 26.9, of 8192 atoms 54.0 /
 // 55.0 / 53.9, of 2048 atoms symmetric 3.90 / 3.90 / 3.11 ms. Within a product the
-// bounds are exact to a 64th, between two of them taken in proportion.
-inline void xcd_split(const WorkParts *const *p, int n, int32_t xcd[kXcds + 1]) {
+// bounds are exact to a 64th, between two of them taken in proportion. At most
+// `at_once` units, which all run at the same time, are split by count where their
+// mean work is at most `brief`: there the fullest compute unit decides.
+inline void xcd_split(const WorkParts *const *p, int n, int32_t at_once, int32_t brief, int32_t xcd[kXcds + 1]) {
+  int32_t total = 0;
+  int64_t work = 0;
+  for (int j = 0; j < n; ++j) {
+    total += p[j]->at[kWorkParts];
+    work += p[j]->work;
+  }
+  if (total <= at_once && work <= (int64_t)total * brief) {
+    const int32_t each = (total + kXcds - 1) / kXcds;
+    for (int x = 0; x <= kXcds; ++x) xcd[x] = std::min(total, x * each);
+    return;
+  }
   double all = 0.0, before = 0.0;
   for (int j = 0; j < n; ++j) all += (double)p[j]->work;
   int32_t base = 0;

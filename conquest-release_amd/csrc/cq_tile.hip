@@ -612,7 +612,7 @@ __global__ void __launch_bounds__(64) k_quad4(const ARG arg) {
   bool nan = false;
 #pragma unroll
   for (int e = 0; e < 4; ++e) nan |= MODE == 1 ? a32[e] != a32[e] : a64[e] != a64[e];
-  if (__ballot(nan) != 0) {
+  if (__builtin_expect(__ballot(nan) != 0, 0)) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       if (MODE == 1 ? a32[e] == a32[e] : a64[e] == a64[e]) continue;
@@ -1420,7 +1420,7 @@ __global__ void __launch_bounds__(kTileThreads) k_tile_dense_mx(
   bool nan = false;
 #pragma unroll
   for (int e = 0; e < 4; ++e) nan |= MODE == 1 ? a32[e] != a32[e] : a64[e] != a64[e];
-  if (__ballot(nan) != 0) {
+  if (__builtin_expect(__ballot(nan) != 0, 0)) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       if (MODE == 1 ? a32[e] == a32[e] : a64[e] == a64[e]) continue;
@@ -1875,12 +1875,21 @@ int tile_group_key(const TilePlan &tp, bool q_trans, int mode) {
   return (tile_kind(tp) * 2 + (q_trans ? 1 : 0)) * 4 + mode;
 }
 
+// Units that are split over the XCDs by count: k_quad4's that fit the card at once
+// (32 wavefronts on each of 256 compute units) and have at most 256 records on
+// average (64 atoms, type 1 8/10/14 A: 27.7 us by work, 26.3 by count). Long units
+// are better split by work at any number (64 atoms, type 2 12/20/28 A: 479 us by
+// work, 515 by count), and so are the other kernels' (32 atoms 16x16, some 3000
+// units: 406 us by work, 484 by count).
+constexpr int32_t kBriefWords = 2048;
+static int32_t units_at_once(const TilePlan &tp) { return tile_kind(tp) == kKindDense4 ? 32 * 256 : 0; }
+
 int launch_tile_args(const TilePlan &tp, bool q_trans, int mode, const TileArgs &a, hipStream_t s) {
   if (a.n_tiles <= 0) return CQMM_OK;
   TileOne one;
   one.a = a;
   const WorkParts *p = &tp.parts;
-  xcd_split(&p, 1, one.xcd);
+  xcd_split(&p, 1, units_at_once(tp), kBriefWords, one.xcd);
   return launch_any(mode, q_trans, tile_kind(tp), one, tp.wgs, s);
 }
 
@@ -1889,7 +1898,7 @@ int launch_tile_group(const TilePlan &tp, bool q_trans, int mode, TileGroup &g, 
   if (g.ngrp > kMaxGroup) return set_errorf(CQMM_ERR_ARG, "grouped tile launch: %d products (at most %d)", g.ngrp, kMaxGroup);
   const WorkParts *p[kMaxGroup];
   for (int j = 0; j < g.ngrp; ++j) p[j] = &g.a[j].plan->parts;
-  xcd_split(p, g.ngrp, g.xcd);
+  xcd_split(p, g.ngrp, units_at_once(tp), kBriefWords, g.xcd);
   return launch_any(mode, q_trans, tile_kind(tp), g, tp.wgs, s);
 }
 

@@ -25,8 +25,8 @@ def split(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-I", CSRC, os.path.join(ROOT, "tests", "xcd_split_driver.cpp"),
                     "-o", str(exe)], check=True, timeout=120)
 
-    def run(works):
-        lines = [str(len(works))]
+    def run(works, at_once=0, brief=0):
+        lines = [f"{len(works)} {at_once} {brief}"]
         for w in works:
             before = np.concatenate(([0], np.cumsum(w)))
             at = [int(np.searchsorted(before, before[-1] / 64 * k)) for k in range(64)] + [len(w)]
@@ -61,6 +61,18 @@ def test_every_xcd_has_its_eighth_of_the_work(split, kind, sizes):
     have = np.diff(before[xcd])
     slack = 2 * unit.max() + (0 if len(works) == 1 else 2 * max(w.sum() for w in works) / 64)
     assert have.max() <= before[-1] / 8 + slack + 1, (have, before[-1] / 8)
+
+
+@pytest.mark.parametrize("sizes", [(1,), (7,), (300,), (5, 3000, 40)])
+def test_brief_units_that_run_at_once_are_split_by_count(split, sizes):
+    works = [_works("heavy", n, np.random.default_rng(n)).astype(np.int64) for n in sizes]
+    total = sum(sizes)
+    each, mean = -(-total // 8), -(-sum(int(w.sum()) for w in works) // total)
+    by_count = np.minimum(np.arange(9) * each, total)
+    np.testing.assert_array_equal(split(works, total, mean), by_count)
+    by_work = split(works)
+    np.testing.assert_array_equal(split(works, total - 1, mean), by_work)
+    np.testing.assert_array_equal(split(works, total, mean - 1), by_work)
 
 
 def test_no_work_at_all(split):
